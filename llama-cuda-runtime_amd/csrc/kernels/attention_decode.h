@@ -76,15 +76,17 @@ __host__ __device__ __forceinline__ void softmax_combine(float* m, float* l, flo
 // positions (64 tiles, so every wave keeps its tiles and their order).
 constexpr int kAttnPositionTable = 4096;
 
-template <bool kPaged, int kHeadDim, int kHeads>
+template <bool kPaged, int kHeadDim, int kHeads, int kWaves = kAttnWaves>
 struct AttnShared {
-  float probs[kAttnWaves][64 * kHeads];
-  float wave_m[kAttnWaves][kHeads];
-  float wave_l[kAttnWaves][kHeads];
-  float wave_acc[kAttnWaves][kHeads][kHeadDim];
+  float probs[kWaves][64 * kHeads];
+  float wave_m[kWaves][kHeads];
+  float wave_l[kWaves][kHeads];
+  float wave_acc[kWaves][kHeads][kHeadDim];
   // Paged layout: the 16-byte-chunk index of position begin + i of the
-  // block's range (chunk 0 of that position's key and value rows).
-  uint32_t chunks[kPaged ? kAttnPositionTable : 1];
+  // block's range (chunk 0 of that position's key and value rows). A block of
+  // fewer waves holds at most one tile per wave.
+  static constexpr int kTable = kWaves == kAttnWaves ? kAttnPositionTable : kWaves * kAttnTile;
+  uint32_t chunks[kPaged ? kTable : 1];
 };
 
 // What a block that runs inside the q/k/v projection's grid takes from it
@@ -178,9 +180,19 @@ using attn_flag = std::integral_constant<bool, B>;
 // queries and the new key and value from exchange words (`x`), and uses the
 // taken key and value in place of the cache's for position seq_len - 1. The
 // arithmetic is unchanged.
-template <bool kPaged, int kHeadDim, int kHeads, bool kExchange = false, typename Prologue = NoPreWait>
+//
+// kWaves: waves of the block, kAttnWaves or, for a range of at most kWaves
+// tiles, 1, 2 or 4. Each wave then has at most one tile, as in the full block,
+// whose other waves merge as (m, l, acc) = (-FLT_MAX, 0, 0): their factor
+// exp(-FLT_MAX - M) is 0 and each fma adds +0 to a sum that is never -0, so
+// leaving them out gives the same bits.
+//
+// Out: where element head * kHeadDim + d of the output goes, an elem_t* or
+// a callable giving a reference.
+template <bool kPaged, int kHeadDim, int kHeads, bool kExchange = false, typename Prologue = NoPreWait,
+          int kWaves = kAttnWaves, typename Out = elem_t*>
 __device__ __forceinline__ void decode_attention_block(
-    AttnShared<kPaged, kHeadDim, kHeads>& sh, elem_t* __restrict__ out,
+    AttnShared<kPaged, kHeadDim, kHeads, kWaves>& sh, Out out,
     float* __restrict__ partials, const elem_t* __restrict__ q, const KvCacheView& view,
     int kv_head, int head0, int split, int splits, int seq_len, float scale,
     const AttnExchange<kHeadDim>* x = nullptr, Prologue prologue = Prologue{}) {
@@ -188,6 +200,9 @@ __device__ __forceinline__ void decode_attention_block(
   constexpr int Q = 64 / P;         // positions per load instruction
   constexpr int G = kHeads;
   static_assert(!kExchange || P <= 8, "exchange blocks take head_dim <= 64");
+  static_assert(kWaves == kAttnWaves || kWaves == 4 || kWaves == 2 || kWaves == 1, "waves of an attention block");
+  constexpr int kThreads = 64 * kWaves;
+  constexpr int kTable = AttnShared<kPaged, kHeadDim, kHeads, kWaves>::kTable;
   const int lane = lane_id();
   const int wave = static_cast<int>(threadIdx.x) >> 6;
   const int j = lane % P;
@@ -203,14 +218,14 @@ __device__ __forceinline__ void decode_attention_block(
   // One thread per page of the window: a single page-table read, then the
   // index of each of the page's positions in the window.
   auto fill_table = [&](int window) {
-    const int window_len = min(kAttnPositionTable, length - window);
+    const int window_len = min(kTable, length - window);
     if (window_len <= 0) return;  // an empty split reads no page-table entry
     const int first = begin + window;                      // first position of the window
     const int first_page = first / view.page_size;
     const int pages = (first + window_len - 1) / view.page_size - first_page + 1;
     const uint32_t head_chunk8 = static_cast<uint32_t>(
         (static_cast<size_t>(kv_head) * static_cast<size_t>(view.head_stride)) / 8);
-    for (int pi = static_cast<int>(threadIdx.x); pi < pages; pi += kAttnThreads) {
+    for (int pi = static_cast<int>(threadIdx.x); pi < pages; pi += kThreads) {
       const int page = first_page + pi;
       const uint32_t base = static_cast<uint32_t>(
           (static_cast<size_t>(view.page_table[page]) * static_cast<size_t>(view.page_stride)) / 8) +
@@ -518,8 +533,8 @@ __device__ __forceinline__ void decode_attention_block(
       load_chunks(view.keys, o, ka);
       load_chunks(view.values, o, va);
       while (true) {
-        const int t1 = tile + kAttnWaves;
-        const bool more1 = t1 < last_tile;
+        const int t1 = tile + kWaves;
+        const bool more1 = kWaves == kAttnWaves && t1 < last_tile;  // fewer waves: one tile each
         if (more1) {
           tile_chunks(t1, window, o);
           load_chunks(view.keys, o, kb);
@@ -532,7 +547,7 @@ __device__ __forceinline__ void decode_attention_block(
         patch_new(tile, ka, va);
         process(tile, ka, va);
         if (!more1) break;
-        const int t2 = t1 + kAttnWaves;
+        const int t2 = t1 + kWaves;
         const bool more2 = t2 < last_tile;
         if (more2) {
           tile_chunks(t2, window, o);
@@ -558,8 +573,8 @@ __device__ __forceinline__ void decode_attention_block(
         if (!x->early_wait) exchange_wait();
       }
       while (true) {
-        const int next = tile + kAttnWaves;
-        const bool more = next < last_tile;
+        const int next = tile + kWaves;
+        const bool more = kWaves == kAttnWaves && next < last_tile;
         const int count = tile_count(tile);
         const bool full = count == kAttnTile;
         patch_new(tile, kr, vr);
@@ -588,7 +603,7 @@ __device__ __forceinline__ void decode_attention_block(
   };
   const int tiles = (length + kAttnTile - 1) / kAttnTile;
   if constexpr (kPaged) {
-    constexpr int kWindowTiles = kAttnPositionTable / kAttnTile;
+    constexpr int kWindowTiles = kTable / kAttnTile;
     if (tiles > 0) run_tiles(0, min(tiles, kWindowTiles), 0, attn_flag<kExchange>{});
     for (int first = kWindowTiles; first < tiles; first += kWindowTiles) {
       __syncthreads();  // every wave is done with the previous window's table
@@ -627,17 +642,17 @@ __device__ __forceinline__ void decode_attention_block(
   // a multiple of 64), and every lane of such a wave takes the maximum of the
   // head's wave maxima; lane w computes c_w, which the wave's lanes read by
   // readlane. No barrier separates the factors from the outputs.
-  static_assert(kHeadDim % 64 == 0 && kAttnWaves <= 64, "a head's outputs are whole waves");
-  for (int idx = threadIdx.x; idx < G * kHeadDim; idx += kAttnThreads) {
+  static_assert(kHeadDim % 64 == 0 && kWaves <= 64, "a head's outputs are whole waves");
+  for (int idx = threadIdx.x; idx < G * kHeadDim; idx += kThreads) {
     const int g = idx / kHeadDim;
     const int d = idx % kHeadDim;
     float tm = sh.wave_m[0][g];
 #pragma unroll
-    for (int v = 1; v < kAttnWaves; ++v) tm = fmaxf(tm, sh.wave_m[v][g]);
-    const float c_lane = lcr_expf(sh.wave_m[lane % kAttnWaves][g] - tm);
+    for (int v = 1; v < kWaves; ++v) tm = fmaxf(tm, sh.wave_m[v][g]);
+    const float c_lane = lcr_expf(sh.wave_m[lane % kWaves][g] - tm);
     float tl = 0.0f, merged = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
       const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c_lane), w));
       tl = __builtin_fmaf(sh.wave_l[w][g], c, tl);
       merged = __builtin_fmaf(c, sh.wave_acc[w][g][d], merged);
@@ -645,7 +660,11 @@ __device__ __forceinline__ void decode_attention_block(
     const int head = head0 + g;
     if (splits == 1) {
       const elem_t e = float_to_elem(merged * (1.0f / tl));
-      out[static_cast<size_t>(head) * kHeadDim + d] = e;
+      if constexpr (std::is_invocable_v<Out, int>) {
+        out(head * kHeadDim + d) = e;
+      } else {
+        out[static_cast<size_t>(head) * kHeadDim + d] = e;
+      }
       if constexpr (kExchange) {
         // kHeadDim is a multiple of 64, so a lane and its odd neighbour hold
         // outputs d and d + 1 of the same wave.

@@ -71,6 +71,24 @@ __device__ __forceinline__ void load_to_lds16(const void* src, uint32_t lds_addr
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds_address) : "memory");
 }
 
+// Wait until at most kCount vector-memory operations of this wave are in
+// flight and every LDS access has returned (gfx9 encoding: vmcnt bits 3:0 and
+// 15:14, expcnt 6:4 left at its maximum, lgkmcnt 11:8 zero).
+template <int kCount>
+__device__ __forceinline__ void wait_stage_landed() {
+  static_assert(kCount >= 0 && kCount < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((kCount & 15) | ((kCount >> 4) << 14) | (7 << 4));
+}
+// The same for LDS accesses alone.
+__device__ __forceinline__ void wait_lds() { wait_stage_landed<63>(); }
+// A barrier that waits for nothing but the block's other waves (loads stay in
+// flight); no memory access moves across it.
+__device__ __forceinline__ void plain_barrier() {
+  asm volatile("" : : : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+}
+
 // LDS byte address of a __shared__ object.
 __device__ __forceinline__ uint32_t lds_address_of(const void* p) {
   typedef const __attribute__((address_space(3))) char* lds_char_ptr;

@@ -687,15 +687,6 @@ __global__ __launch_bounds__(64 * kWavesW * kWavesT) void gemm_nt_kernel(
 // count waits stricter.
 constexpr int kRingK = 32;
 
-// Wait until at most kCount vector-memory operations of this wave are in
-// flight and every LDS read has returned (gfx9 encoding: vmcnt bits 3:0 and
-// 15:14, expcnt 6:4 left at its maximum, lgkmcnt 11:8 zero).
-template <int kCount>
-__device__ __forceinline__ void wait_stage_landed() {
-  static_assert(kCount >= 0 && kCount < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((kCount & 15) | ((kCount >> 4) << 14) | (7 << 4));
-}
-
 // Block tiles of BW W rows x BT tokens:
 //  - 256 x 256, kWaves = 8: wave tiles of 128 W rows x 64 tokens (two waves
 //    per SIMD);
@@ -958,7 +949,7 @@ __global__ __launch_bounds__(kNormThreads) void gemm_reduce_norm_kernel(const fl
   const size_t base = static_cast<size_t>(blockIdx.x) * dim;
   const size_t count = static_cast<size_t>(T) * dim;
   norm_row_vec<true, kChunks>(
-      n.out + base, n.x + base, n.weight, dim, n.eps,
+      [&](int c) { return n.out + base + 8 * c; }, n.x + base, n.weight, dim, n.eps,
       [&](int c, float* df) {
         const float* p = partial + base + 8 * c;
         float4 a = *reinterpret_cast<const float4*>(p);

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(elem_t* __res
   __shared__ float scratch[9];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * dim;
   norm_row_vec<kResidual, kChunks>(
-      out + base, x + base, weight, dim, eps,
+      [&](int c) { return out + base + 8 * c; }, x + base, weight, dim, eps,
       [&](int c, float* df) { unpack8(load16(delta + base + 8 * c), df); }, scratch);
 }
 

@@ -72,9 +72,10 @@ __device__ __forceinline__ float norm_scale(float total, int dim, float eps) {
 // elements with at most kChunks chunks per thread: thread t holds chunks
 // t, t + 256, ... (the order block_sum_squares walks), so the sum of squares
 // and the roundings are those of block_sum_squares' element loop, bit for bit.
-// delta(c, df) writes the eight addends of chunk c to df[0..7].
-template <bool kResidual, int kChunks, typename Delta>
-__device__ __forceinline__ void norm_row_vec(elem_t* __restrict__ orow, elem_t* __restrict__ xrow,
+// delta(c, df) writes the eight addends of chunk c to df[0..7]; out_chunk(c)
+// is where chunk c of the output goes.
+template <bool kResidual, int kChunks, typename OutChunk, typename Delta>
+__device__ __forceinline__ void norm_row_vec(OutChunk out_chunk, elem_t* __restrict__ xrow,
                                              const elem_t* __restrict__ weight, int dim, float eps,
                                              Delta delta, float* scratch) {
   const int chunks = dim / 8;
@@ -120,7 +121,7 @@ __device__ __forceinline__ void norm_row_vec(elem_t* __restrict__ orow, elem_t* 
       const float b = elem_bits_to_float(float_to_elem_bits(v[k][2 * j + 1]));
       r.w[j] = pack_elems((a * scale) * wf[2 * j], (b * scale) * wf[2 * j + 1]);
     }
-    store16(orow + 8 * c, r);
+    store16(out_chunk(c), r);
   }
 }
 

@@ -8,6 +8,7 @@
 #include "hip_utils.h"
 #include "kernels.h"
 #include "kernels/fill.h"
+#include "kernels/short_prompt.h"
 
 namespace lcr {
 namespace {
@@ -213,6 +214,14 @@ void Model::allocate_arena() {
   const size_t attn_floats = std::max<size_t>(
       decode_attention_scratch_floats(config_.num_heads, config_.head_dim, kMaxAttentionSplits),
       sample_scratch_floats(config_.vocab_size, 0));
+  // Short chunks' projection inputs and sums, where those kernels can run.
+  const int short_tokens = decode_step_supported(config_.hidden_size, config_.intermediate_size, config_.num_heads,
+                                                 config_.num_kv_heads, config_.head_dim)
+                               ? std::min(max_tokens_, kMinMfmaPrefillTokens - 1)
+                               : 0;
+  const size_t short_hidden = short_fragment_elements(short_tokens, config_.hidden_size);
+  const size_t short_ffn = short_fragment_elements(short_tokens, config_.intermediate_size);
+  const size_t short_sums = short_partial_floats(short_tokens, config_.hidden_size, config_.intermediate_size);
   const size_t sizes[] = {
       T * H * e,                                 // x_
       T * H * e,                                 // normed_
@@ -235,6 +244,10 @@ void Model::allocate_arena() {
       sizeof(int32_t),                                                // draw_counter_
       decode_exchange_words(config_.num_heads, config_.head_dim) * sizeof(unsigned long long),  // exchange_words_
       sizeof(uint32_t),                                               // epoch_
+      short_hidden * e,                                               // short_normed_
+      short_hidden * e,                                               // short_attn_
+      short_ffn * e,                                                  // short_act_
+      short_sums * sizeof(float),                                     // short_partial_
   };
   size_t total = 0;
   for (size_t s : sizes) total = align_up(total, 256) + s;
@@ -262,6 +275,12 @@ void Model::allocate_arena() {
   draw_counter_ = arena_.alloc<int32_t>(1);
   exchange_words_ = arena_.alloc<unsigned long long>(decode_exchange_words(config_.num_heads, config_.head_dim));
   epoch_ = arena_.alloc<uint32_t>(1);
+  if (short_tokens > 0) {
+    short_normed_ = arena_.alloc<elem_t>(short_hidden);
+    short_attn_ = arena_.alloc<elem_t>(short_hidden);
+    short_act_ = arena_.alloc<elem_t>(short_ffn);
+    short_partial_ = arena_.alloc<float>(short_sums);
+  }
   HIP_CHECK(hipMemset(epoch_, 0, sizeof(uint32_t)));
   clear_exchange();
   HIP_CHECK(hipMemset(token_ids_, 0, T * sizeof(int32_t)));
@@ -329,6 +348,11 @@ const float* Model::prefill(const std::vector<int>& tokens) {
   while (consumed < tokens.size()) {
     const int chunk = static_cast<int>(std::min<size_t>(static_cast<size_t>(max_tokens_),
                                                         tokens.size() - consumed));
+    if (runs_as_short_prompt(chunk)) {
+      prefill_short(tokens.data() + consumed, chunk);
+      consumed += static_cast<size_t>(chunk);
+      continue;
+    }
     if (chunk < kMinMfmaPrefillTokens) {
       for (int i = 0; i < chunk; ++i) decode(tokens[consumed + static_cast<size_t>(i)]);
       consumed += static_cast<size_t>(chunk);
@@ -353,6 +377,67 @@ const float* Model::prefill(const std::vector<int>& tokens) {
   stats_.last_prefill_ms = timer.elapsed_ms();
   if (profiler_.enabled()) profiler_.collect();
   return logits_;
+}
+
+// The kernels of short_prompt.h cover the fused step's geometries, one
+// attention split, and chunks of two tokens up: one token is the step itself.
+// Captured activations are those of single steps.
+bool Model::runs_as_short_prompt(int chunk) const {
+  return fused_ && !capture_activations_ && chunk > 1 && chunk < kMinMfmaPrefillTokens &&
+         decode_splits(position_ + chunk) == 1;
+}
+
+// decode() of each token, with the weights streamed once for all of them: the
+// layers of the whole chunk, then the fused step's output head on the last
+// token, which leaves the step state and the logits as that token's decode()
+// would.
+void Model::prefill_short(const int* tokens, int count) {
+  HIP_CHECK(hipMemcpyAsync(token_ids_, tokens, static_cast<size_t>(count) * sizeof(int32_t), hipMemcpyHostToDevice,
+                           stream_));
+  kv_cache_->reserve_length(position_ + count);
+  ShortPromptArgs a{};
+  a.tokens = count;
+  a.position = position_;
+  a.num_heads = config_.num_heads;
+  a.num_kv_heads = config_.num_kv_heads;
+  a.head_dim = config_.head_dim;
+  a.hidden = config_.hidden_size;
+  a.ffn = config_.intermediate_size;
+  a.compute_units = multiprocessors_;
+  a.paged = options_.kv_layout == KvLayout::kPaged;
+  a.rope_table = rope_table_;
+  a.x = x_;
+  a.q = q_heads_;
+  a.normed = short_normed_;
+  a.attn = short_attn_;
+  a.act = short_act_;
+  a.partial = short_partial_;
+  const int slices = short_down_slices(a.ffn);
+  const float eps = config_.rms_norm_eps;
+  for (int layer = 0; layer < config_.num_layers; ++layer) {
+    const LayerWeights& lw = layers_[static_cast<size_t>(layer)];
+    const LayerDevicePtrs w{lw.input_norm, lw.qkv_proj, lw.o_proj, lw.post_attention_norm,
+                            lw.gate_up_proj, lw.down_proj};
+    if (layer == 0) {
+      enqueue_short_embed_norm(a, embedding_, token_ids_, w.input_norm, eps, stream_);
+    } else {
+      enqueue_short_residual_norm(a, w.input_norm, slices, eps, stream_);
+    }
+    enqueue_short_qkv_attention(a, w, kv_cache_->view(layer), stream_);
+    enqueue_short_oproj(a, w, stream_);
+    enqueue_short_residual_norm(a, w.post_norm, 1, eps, stream_);
+    enqueue_short_mlp(a, w, stream_);
+  }
+  enqueue_short_residual(a, resid_, stream_);
+  position_ += count - 1;
+  write_step_state(tokens[count - 1], true);
+  enqueue_decode_head(step_args(1), stream_);
+  position_ += 1;
+  HIP_CHECK(hipStreamSynchronize(stream_));
+  check_exchange();
+  device_token_ = __atomic_load_n(step_id_host_, __ATOMIC_ACQUIRE);
+  step_argmax_ready_ = true;
+  step_state_current_ = true;
 }
 
 // want_host_id: the step's output head also writes its greedy id to

@@ -85,9 +85,9 @@ class Model {
     bool exchange_head = true;
   };
 
-  // Prompt chunks shorter than this run token by token through the decode
-  // step (GEMV path, bit-identical to decoding them) rather than through the
-  // MFMA GEMMs, which only pay off from a few tiles of tokens upward.
+  // Prompt chunks shorter than this give every token the bits of decoding it
+  // (kernels/short_prompt.h, or the decode step token by token where those
+  // kernels do not run) rather than running through the MFMA GEMMs.
   static constexpr int kMinMfmaPrefillTokens = 64;
 
   Model(const std::string& model_dir, const Options& options);
@@ -186,6 +186,8 @@ class Model {
   void capture_f32_residual(const std::string& name);
   void write_step_state(int token, bool want_host_id);
   void enqueue_fused_step();
+  bool runs_as_short_prompt(int chunk) const;
+  void prefill_short(const int* tokens, int count);
   void launch_fused_step(int seq_len);
   DecodeStepArgs step_args(int splits) const;
   void advance_epoch();
@@ -224,6 +226,11 @@ class Model {
   float* attention_scratch_ = nullptr;
   float* gemm_workspace_ = nullptr;  // split-K partial products of the prefill projections
   size_t gemm_workspace_size_ = 0;
+  // Short prompt chunks (kernels/short_prompt.h).
+  elem_t* short_normed_ = nullptr;
+  elem_t* short_attn_ = nullptr;
+  elem_t* short_act_ = nullptr;
+  float* short_partial_ = nullptr;
   int32_t* token_ids_ = nullptr;  // [max_tokens]
   int32_t* sampled_id_ = nullptr;
   // Fused decode state.
