@@ -76,16 +76,15 @@ __host__ __device__ __forceinline__ void softmax_combine(float* m, float* l, flo
 // positions (64 tiles, so every wave keeps its tiles and their order).
 constexpr int kAttnPositionTable = 4096;
 
-template <bool kPaged, int kHeadDim, int kHeads, int kWaves = kAttnWaves>
+template <bool kPaged, int kHeadDim, int kHeads, int kWaves = kAttnWaves, bool kOneTile = (kWaves < kAttnWaves)>
 struct AttnShared {
   float probs[kWaves][64 * kHeads];
   float wave_m[kWaves][kHeads];
   float wave_l[kWaves][kHeads];
   float wave_acc[kWaves][kHeads][kHeadDim];
   // Paged layout: the 16-byte-chunk index of position begin + i of the
-  // block's range (chunk 0 of that position's key and value rows). A block of
-  // fewer waves holds at most one tile per wave.
-  static constexpr int kTable = kWaves == kAttnWaves ? kAttnPositionTable : kWaves * kAttnTile;
+  // block's range (chunk 0 of that position's key and value rows).
+  static constexpr int kTable = kOneTile ? kWaves * kAttnTile : kAttnPositionTable;
   uint32_t chunks[kPaged ? kTable : 1];
 };
 
@@ -181,18 +180,20 @@ using attn_flag = std::integral_constant<bool, B>;
 // taken key and value in place of the cache's for position seq_len - 1. The
 // arithmetic is unchanged.
 //
-// kWaves: waves of the block, kAttnWaves or, for a range of at most kWaves
-// tiles, 1, 2 or 4. Each wave then has at most one tile, as in the full block,
-// whose other waves merge as (m, l, acc) = (-FLT_MAX, 0, 0): their factor
-// exp(-FLT_MAX - M) is 0 and each fma adds +0 to a sum that is never -0, so
-// leaving them out gives the same bits.
+// kOneTile: the range has at most kWaves tiles, so a wave holds no registers
+// for a second one (G = 1: 123 to 152 VGPRs instead of 240, twice the blocks on
+// a compute unit).
+// kWaves: waves of the block, kAttnWaves or, with kOneTile, 1, 2 or 4. The full
+// block's other waves would merge as (m, l, acc) = (-FLT_MAX, 0, 0): their
+// factor exp(-FLT_MAX - M) is 0 and each fma adds +0 to a sum that is never
+// -0, so leaving them out gives the same bits.
 //
 // Out: where element head * kHeadDim + d of the output goes, an elem_t* or
 // a callable giving a reference.
 template <bool kPaged, int kHeadDim, int kHeads, bool kExchange = false, typename Prologue = NoPreWait,
-          int kWaves = kAttnWaves, typename Out = elem_t*>
+          int kWaves = kAttnWaves, typename Out = elem_t*, bool kOneTile = (kWaves < kAttnWaves)>
 __device__ __forceinline__ void decode_attention_block(
-    AttnShared<kPaged, kHeadDim, kHeads, kWaves>& sh, Out out,
+    AttnShared<kPaged, kHeadDim, kHeads, kWaves, kOneTile>& sh, Out out,
     float* __restrict__ partials, const elem_t* __restrict__ q, const KvCacheView& view,
     int kv_head, int head0, int split, int splits, int seq_len, float scale,
     const AttnExchange<kHeadDim>* x = nullptr, Prologue prologue = Prologue{}) {
@@ -202,7 +203,8 @@ __device__ __forceinline__ void decode_attention_block(
   static_assert(!kExchange || P <= 8, "exchange blocks take head_dim <= 64");
   static_assert(kWaves == kAttnWaves || kWaves == 4 || kWaves == 2 || kWaves == 1, "waves of an attention block");
   constexpr int kThreads = 64 * kWaves;
-  constexpr int kTable = AttnShared<kPaged, kHeadDim, kHeads, kWaves>::kTable;
+  static_assert(kOneTile || kWaves == kAttnWaves, "fewer waves hold one tile each");
+  constexpr int kTable = AttnShared<kPaged, kHeadDim, kHeads, kWaves, kOneTile>::kTable;
   const int lane = lane_id();
   const int wave = static_cast<int>(threadIdx.x) >> 6;
   const int j = lane % P;
@@ -534,7 +536,7 @@ __device__ __forceinline__ void decode_attention_block(
       load_chunks(view.values, o, va);
       while (true) {
         const int t1 = tile + kWaves;
-        const bool more1 = kWaves == kAttnWaves && t1 < last_tile;  // fewer waves: one tile each
+        const bool more1 = !kOneTile && t1 < last_tile;
         if (more1) {
           tile_chunks(t1, window, o);
           load_chunks(view.keys, o, kb);
@@ -574,7 +576,7 @@ __device__ __forceinline__ void decode_attention_block(
       }
       while (true) {
         const int next = tile + kWaves;
-        const bool more = kWaves == kAttnWaves && next < last_tile;
+        const bool more = !kOneTile && next < last_tile;
         const int count = tile_count(tile);
         const bool full = count == kAttnTile;
         patch_new(tile, kr, vr);

@@ -20,14 +20,16 @@
 namespace lcr {
 namespace {
 
-// One block per (query head, split); query head h reads kv head h / kGroup.
-template <bool kPaged, int kHeadDim, int kGroup>
-__global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
+// One block of kWaves waves per (kHeads query heads, split); query head h
+// reads kv head h / group.
+template <bool kPaged, int kHeadDim, int kHeads, int kWaves, bool kOneTile>
+__global__ __launch_bounds__(64 * kWaves) void decode_attention_kernel(
     elem_t* __restrict__ out, float* __restrict__ partials, const elem_t* __restrict__ q,
-    KvCacheView view, int seq_len, float scale, int splits) {
-  __shared__ AttnShared<kPaged, kHeadDim, 1> sh;
-  decode_attention_block<kPaged, kHeadDim, 1>(sh, out, partials, q, view, blockIdx.x / kGroup,
-                                           blockIdx.x, blockIdx.y, splits, seq_len, scale);
+    KvCacheView view, int group, int seq_len, float scale, int splits) {
+  __shared__ AttnShared<kPaged, kHeadDim, kHeads, kWaves, kOneTile> sh;
+  const int head0 = static_cast<int>(blockIdx.x) * kHeads;
+  decode_attention_block<kPaged, kHeadDim, kHeads, false, NoPreWait, kWaves, elem_t*, kOneTile>(
+      sh, out, partials, q, view, head0 / group, head0, blockIdx.y, splits, seq_len, scale);
 }
 
 __global__ __launch_bounds__(kMergeThreads) void merge_splits_kernel(elem_t* __restrict__ out,
@@ -131,12 +133,46 @@ struct DecodeArgs {
   hipStream_t stream;
 };
 
+template <bool kPaged, int kHeadDim, int kHeads, int kWaves, bool kOneTile>
+int launch_blocks(int group, const DecodeArgs& a) {
+  const dim3 grid(static_cast<unsigned>(a.num_heads / kHeads), static_cast<unsigned>(a.splits));
+  decode_attention_kernel<kPaged, kHeadDim, kHeads, kWaves, kOneTile><<<grid, 64 * kWaves, 0, a.stream>>>(
+      a.out, a.partials, a.q, a.view, group, a.seq_len, a.scale, a.splits);
+  CAPI_LAUNCHED();
+  return LCR_OK;
+}
+
+// The block for the tiles of a split (the same bits from each): as many waves
+// as tiles up to eight, and registers for a second tile only where a wave has
+// one. One split of 40 positions at head_dim 128: 8.6 -> 5.4 us; 32 splits of
+// 256 positions, per head, head_dim 64: 24.6 -> 17.3 us.
+template <bool kPaged, int kHeadDim, int kHeads>
+int launch_waves(int group, const DecodeArgs& a) {
+  const int tiles = ((a.seq_len + a.splits - 1) / a.splits + kAttnTile - 1) / kAttnTile;
+  if constexpr (kHeads == 1) {
+    if (tiles <= 1) return launch_blocks<kPaged, kHeadDim, kHeads, 1, true>(group, a);
+    if (tiles <= 2) return launch_blocks<kPaged, kHeadDim, kHeads, 2, true>(group, a);
+  }
+  if (tiles <= 4) return launch_blocks<kPaged, kHeadDim, kHeads, 4, true>(group, a);
+  if (tiles <= kAttnWaves) return launch_blocks<kPaged, kHeadDim, kHeads, kAttnWaves, true>(group, a);
+  return launch_blocks<kPaged, kHeadDim, kHeads, kAttnWaves, false>(group, a);
+}
+
+// From this many splits on, one block serves up to four query heads of a kv
+// head, reading each key and value once for them. Below, per-head blocks fill
+// the device better: 11 splits (3000 positions) take 11.0 us per head against
+// 12.2 shared at head_dim 64, 11.8 against 12.3 at 128; 16 splits (4096) 11.5
+// against 10.6 and 13.2 against 11.3; 64 splits (32768, paged) 52.5 against
+// 26.6 and 51.1 against 38.2.
+constexpr int kSharedHeadsMinSplits = 16;
+
 template <bool kPaged, int kHeadDim, int kGroup>
 int launch_decode(const DecodeArgs& a) {
-  const dim3 grid(static_cast<unsigned>(a.num_heads), static_cast<unsigned>(a.splits));
-  decode_attention_kernel<kPaged, kHeadDim, kGroup><<<grid, kAttnThreads, 0, a.stream>>>(
-      a.out, a.partials, a.q, a.view, a.seq_len, a.scale, a.splits);
-  CAPI_LAUNCHED();
+  constexpr int kShared = kGroup < 4 ? kGroup : 4;
+  const int status = kShared > 1 && a.splits >= kSharedHeadsMinSplits
+                         ? launch_waves<kPaged, kHeadDim, kShared>(kGroup, a)
+                         : launch_waves<kPaged, kHeadDim, 1>(kGroup, a);
+  if (status != LCR_OK) return status;
   if (a.splits > 1) {
     merge_splits_kernel<<<a.num_heads, kMergeThreads, 0, a.stream>>>(a.out, a.partials, a.splits, kHeadDim);
     CAPI_LAUNCHED();
