@@ -18,17 +18,16 @@
 // lcr_prefill_attention replaces the reference's gather + two strided-batched
 // GEMMs + causal softmax (src/model.cu:509-560; src/kernels/attention.cu:42-100).
 // Query row r of the chunk sits at position start + r and sees keys
-// 0..start+r; scores are (q . k) * scale in fp32. A block takes 16*RF
-// positions of the query heads that share one kv head (four per block, one
-// wave each) and walks 64-key tiles of that kv head staged in LDS (double
-// buffered). Each wave computes S^T = K . Q^T, so an accumulator lane holds
-// one query row and 4 keys: a row statistic needs two lane exchanges, and the
-// probabilities are already in the operand layout of O^T = V^T . P^T (V is
-// staged transposed). The softmax follows the reference's rounding points: a
-// first pass over the keys finds each row's max M and sum L of exp(s - M),
-// the second forms p = exp(s - M) * (1/L), rounds it to the element type (the
-// reference's probability buffer) and accumulates p * v in fp32, rounded once
-// on store.
+// 0..start+r; scores are (q . k) * scale in fp32. A block takes 16 or 32
+// positions of the query heads that share one kv head (four per block), a wave
+// per head and key group, and walks 64-key tiles of that kv head staged in LDS.
+// Each wave computes S^T = K . Q^T, so an accumulator lane holds one query row
+// and 4 keys: a row statistic needs two lane exchanges, and the probabilities
+// are already in the operand layout of O^T = V^T . P^T. The softmax follows
+// the reference's rounding points: a first pass over the keys finds each row's
+// max M and sum L of exp(s - M), the second forms p = exp(s - M) / L, rounds
+// it to the element type (the reference's probability buffer) and accumulates
+// p * v in fp32, rounded once on store.
 #include <algorithm>
 
 #include "../capi_util.h"
@@ -1182,13 +1181,11 @@ bool run_gemm(void* Y, bool fp32_out, const elem_t* X, const elem_t* W, int T, i
 // Prefill attention (MFMA, flash-style)
 // ---------------------------------------------------------------------------
 
-// Eight waves: the four query heads of one kv head, each over two key groups
-// (the even and the odd 64-key tiles), so a block walks its keys in half the
-// steps; the two groups merge their statistics and their outputs at fixed
-// points, group 0 first.
-constexpr int kFlashThreads = 512;
-constexpr int kFlashKeys = 64;      // keys per tile; two tiles are staged per step
-constexpr int kKeyGroups = 2;
+// A wave per (query head of a kv head, key group): a block serves four heads,
+// and group k of kKG walks the 64-key tiles k, k + kKG, ..., so that a step
+// stages kKG tiles. The groups merge their statistics and their outputs at
+// fixed points, group 0 first.
+constexpr int kFlashKeys = 64;  // keys per tile
 
 // Key rows are head_dim elements with 16-byte chunk c at position
 // c ^ key_swizzle(key), so the fragment reads of 16 consecutive keys are free
@@ -1211,48 +1208,61 @@ __device__ __forceinline__ int value_swizzle(int key) {
   return kHeadDim == 64 ? (key & 6) : ((key & 7) << 1);
 }
 
-template <int kHeadDim, int kRows>
+template <int kHeadDim, int kRows, int kKG>
 struct FlashShared {
-  static constexpr int kKeyPitch = kHeadDim;
-  elem_t keys[2][kKeyGroups * kFlashKeys * kKeyPitch];    // two tiles per buffer
-  elem_t values[2][kKeyGroups * kFlashKeys * kHeadDim];   // the same keys' values
-  float stats[kFlashThreads / 64][kRows][2];              // per wave: row max, row sum
+  // Pass 1 stages keys alone, through all four buffers; pass 2 keys in the
+  // first two and the same keys' values in the others.
+  elem_t tiles[4][kKG * kFlashKeys * kHeadDim];
+  float stats[4 * kKG][kRows][2];  // per wave: row max, row sum
 };
 
 typedef short lds_v4i16 __attribute__((ext_vector_type(4)));
 
-template <bool kPaged, int kHeadDim, int kRF>
-__global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_prefill_kernel(
+// Bound by VALU work (16 exponentials a lane and tile in each pass, each at a
+// quarter of the rate) and, next to it, by LDS reads of the tiles with 16 rows a
+// wave. Pass 1 runs three steps ahead of its loads through all four buffers,
+// keeps its maximum and sum per lane, and pass 2 takes 1 / L inside the
+// exponent: with the page entries below, T = 2048 paged 58.8 -> 52.0 us, T =
+// 500 at 6144 paged 105 -> 87 (16 rows, two key groups on both sides). One pass
+// with the weights as two elements took 40 us at T = 2048 and 61 at T = 500,
+// closer to float64, but does not round the probabilities where the reference
+// does.
+template <bool kPaged, int kHeadDim, int kRF, int kKG>
+__global__ __launch_bounds__(256 * kKG, kHeadDim == 64 ? 4 : 2) void flash_prefill_kernel(
     elem_t* __restrict__ out, const elem_t* __restrict__ q_heads, KvCacheView view, int num_heads,
-    int group, int tokens, int start_position, float scale_log2e) {
+    int group, int tokens, int start_position, float scale_log2e, bool folded) {
+  constexpr int kWaves = 4 * kKG;
   constexpr int kRows = 16 * kRF;                         // query positions per block
   constexpr int kSteps = kHeadDim / 32;                   // MFMA k-steps over head_dim
   constexpr int kDFrags = kHeadDim / 16;                  // output fragments over head_dim
-  constexpr int kPairKeys = kKeyGroups * kFlashKeys;      // keys staged per step
-  constexpr int kKeyPitch = FlashShared<kHeadDim, kRows>::kKeyPitch;
+  constexpr int kStepKeys = kKG * kFlashKeys;             // keys staged per step
   constexpr int kRowChunks = kHeadDim / 8;                // 16-byte chunks per key row
   constexpr int kLoadRows = 64 / kRowChunks;              // rows of one 1 KiB direct load
-  constexpr int kWaveLoads = kPairKeys / kLoadRows / (kFlashThreads / 64);  // per wave, K or V
-  static_assert(kWaveLoads * kLoadRows * (kFlashThreads / 64) == kPairKeys, "a step splits over the waves");
-  static_assert(kKeyGroups * 4 == kFlashThreads / 64, "one wave per (head, key group)");
-  __shared__ __attribute__((aligned(1024))) FlashShared<kHeadDim, kRows> sh;
+  constexpr int kWaveLoads = kStepKeys / kLoadRows / kWaves;  // per wave, K or V
+  static_assert(kWaveLoads * kLoadRows * kWaves == kStepKeys, "a step splits over the waves");
+  using Shared = FlashShared<kHeadDim, kRows, kKG>;
+  __shared__ __attribute__((aligned(1024))) Shared sh;
 
   // XCD-aware order: XCD x (block id mod 8) takes the contiguous run of units
   // [x * per, (x + 1) * per) of the kv-head-major order, so one XCD's L2 holds
-  // the keys and values of few kv heads (one, for 8 kv heads); within a head,
-  // the longest rows start first.
+  // the keys and values of few kv heads (one, for 8 kv heads). Within a head
+  // the longest rows start first; `folded`, only the longer half does, and the
+  // shorter half follows from the shortest up, so that the two blocks of a
+  // compute unit (dispatched round robin) have the same work in sum.
   const int row_blocks = (tokens + kRows - 1) / kRows;
   const int units = row_blocks * view.num_kv_heads;
   const int per_xcd = (units + 7) / 8;
   const int u = static_cast<int>(blockIdx.x % 8u) * per_xcd + static_cast<int>(blockIdx.x / 8u);
   if (u >= units) return;  // the whole block: no barrier has been met
   const int kv = u / row_blocks;
-  const int r0 = (row_blocks - 1 - u % row_blocks) * kRows;
+  const int place = u % row_blocks;
+  const int longer = (row_blocks + 1) / 2;
+  const int r0 = (folded && place >= longer ? place - longer : row_blocks - 1 - place) * kRows;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = lane_id();
   const int col = lane & 15;
   const int grp = lane >> 4;
-  const int kg = wave >> 2;  // key group: tiles kg, kg + 2, ...
+  const int kg = wave >> 2;  // key group: tiles kg, kg + kKG, ...
   const int g = blockIdx.z * 4 + (wave & 3);
   const bool active = g < group;
   const int head = kv * group + (active ? g : 0);
@@ -1260,7 +1270,7 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
   const int last_key = start_position + tokens - 1;
   const int block_keys = start_position + min(r0 + kRows, tokens);
   const int tiles = (block_keys + kFlashKeys - 1) / kFlashKeys;
-  const int steps = (tiles + kKeyGroups - 1) / kKeyGroups;
+  const int steps = (tiles + kKG - 1) / kKG;
 
   // Q fragments, the N side of S^T: row r0 + 16rf + col, dims 32ks + 8grp .. +7.
   mfma_in8 qf[kRF][kSteps];
@@ -1277,25 +1287,58 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
     }
   }
 
-  // Step `step` stages tiles 2 step and 2 step + 1 (keys 128 step .. +127)
-  // by direct global-to-LDS loads, no registers between: load n of a wave
-  // fills rows kLoadRows (8 n + wave) .. + kLoadRows - 1, lane i writing slot
+  // Step `step` stages its kKG tiles (keys kStepKeys step ..) by direct
+  // global-to-LDS loads, no registers between: load n of a wave fills rows
+  // kLoadRows (kWaves n + wave) .. + kLoadRows - 1, lane i writing slot
   // i % kRowChunks of row i / kRowChunks, so the lane loads the chunk whose
   // swizzled position that slot is. Keys past the last position repeat it (the
   // scores mask them).
+  //
+  // Paged: with power-of-two pages of at least a load's rows, a load lies in
+  // one page, whose table entry is a scalar load made a step ahead. A vector
+  // load of it would be waited for with every tile load in flight (loads
+  // complete in order).
   const int load_row = lane / kRowChunks;
   const int load_slot = lane % kRowChunks;
-  auto issue = [&](int step, int buf, bool with_values) {
+  const bool whole_pages = kPaged && view.page_size >= kLoadRows && (view.page_size & (view.page_size - 1)) == 0;
+  const int page_shift = whole_pages ? 31 - __builtin_clz(view.page_size) : 0;
+  struct StepPages {
+    int32_t page[kWaveLoads];
+  };
+  auto pages_of = [&](int step) {
+    StepPages pages{};
+    if constexpr (kPaged) {
+      if (whole_pages) {
+        typedef const __attribute__((address_space(4))) int32_t* constant_ptr;
+        const constant_ptr table = (constant_ptr)(reinterpret_cast<uintptr_t>(view.page_table));
+#pragma unroll
+        for (int n = 0; n < kWaveLoads; ++n) {
+          const int key = min(step * kStepKeys + kLoadRows * (kWaves * n + wave), last_key);
+          pages.page[n] = table[__builtin_amdgcn_readfirstlane(key >> page_shift)];
+        }
+      }
+    }
+    return pages;
+  };
+  auto issue = [&](int step, const StepPages& pages, elem_t* keys, elem_t* values) {
 #pragma unroll
     for (int n = 0; n < kWaveLoads; ++n) {
-      const int block_row = kLoadRows * (8 * n + wave);
+      const int block_row = kLoadRows * (kWaves * n + wave);
       const int row = block_row + load_row;
-      const size_t at = view.offset<kPaged>(kv, min(step * kPairKeys + row, last_key));
+      const int key = min(step * kStepKeys + row, last_key);
+      size_t at;
+      if (kPaged && whole_pages) {
+        at = static_cast<size_t>(pages.page[n]) * static_cast<size_t>(view.page_stride) +
+             static_cast<size_t>(kv) * static_cast<size_t>(view.head_stride) +
+             static_cast<size_t>((key & (view.page_size - 1)) * kHeadDim);
+      } else {
+        at = view.offset<kPaged>(kv, key);
+      }
       load_to_lds16(view.keys + at + 8 * (load_slot ^ key_swizzle<kHeadDim>(row)),
-                    lds_address_of(&sh.keys[buf][block_row * kKeyPitch]));
-      if (with_values) {
+                    lds_address_of(keys + block_row * kHeadDim));
+      if (values != nullptr) {
         load_to_lds16(view.values + at + 8 * (load_slot ^ value_swizzle<kHeadDim>(row)),
-                      lds_address_of(&sh.values[buf][block_row * kHeadDim]));
+                      lds_address_of(values + block_row * kHeadDim));
       }
     }
   };
@@ -1324,8 +1367,8 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
   // `tile`; keys past a row's position are -inf. The scale (in base-2 units,
   // scale * log2(e)) is applied inside the exponentials, as one fma with the
   // row max: exp2(c s - c m).
-  auto scores = [&](int buf, int tile, mfma_acc4 (&s)[kRF][4]) {
-    const elem_t* kb = &sh.keys[buf][kg * kFlashKeys * kKeyPitch];
+  auto scores = [&](const elem_t* keys, int tile, mfma_acc4 (&s)[kRF][4]) {
+    const elem_t* kb = keys + kg * kFlashKeys * kHeadDim;
 #pragma unroll
     for (int kf = 0; kf < 4; ++kf) {
 #pragma unroll
@@ -1333,7 +1376,7 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
 #pragma unroll
       for (int ks = 0; ks < kSteps; ++ks) {
         const mfma_in8 a = lds_operand(
-            kb + (kf * 16 + col) * kKeyPitch + (((ks * 4 + grp) ^ key_swizzle<kHeadDim>(col)) << 3));
+            kb + (kf * 16 + col) * kHeadDim + (((ks * 4 + grp) ^ key_swizzle<kHeadDim>(col)) << 3));
 #pragma unroll
         for (int rf = 0; rf < kRF; ++rf) s[rf][kf] = mfma16x16x32(a, qf[rf][ks], s[rf][kf]);
       }
@@ -1354,38 +1397,47 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
     }
   };
 
-  // Pass 1: per key group, row max m and sum l of exp(s - m), keys only; the
-  // sum is kept per lane against a running max and rescaled when it grows.
+  // Pass 1: row max m and sum l of exp(s - m), keys only. Each lane keeps the
+  // max and the sum of its own keys (4 of each 16), the sum rescaled when the
+  // max grows; lanes and key groups merge after the last tile.
   float m[kRF], l[kRF];
 #pragma unroll
   for (int rf = 0; rf < kRF; ++rf) {
     m[rf] = -__builtin_huge_valf();
     l[rf] = 0.0f;
   }
-  issue(0, 0, false);
-  wait_stage_landed<0>();
-  __syncthreads();
+  {
+    const StepPages p0 = pages_of(0), p1 = pages_of(1), p2 = pages_of(2);
+    issue(0, p0, sh.tiles[0], nullptr);
+    if (1 < steps) issue(1, p1, sh.tiles[1], nullptr);
+    if (2 < steps) issue(2, p2, sh.tiles[2], nullptr);
+  }
+  StepPages pages = pages_of(3);
   for (int step = 0; step < steps; ++step) {
-    const int buf = step & 1;
-    // buf ^ 1 was last read in the previous step, before its closing barrier
-    if (step + 1 < steps) issue(step + 1, buf ^ 1, false);
-    const int tile = kKeyGroups * step + kg;
+    // This wave's loads of the step have landed (at most the two younger
+    // steps' remain); after the barrier every wave's have, and the buffer of
+    // the step before is free.
+    if (step + 2 < steps) {
+      wait_stage_landed<2 * kWaveLoads>();
+    } else {
+      wait_stage_landed<0>();
+    }
+    plain_barrier();
+    if (step + 3 < steps) issue(step + 3, pages, sh.tiles[(step + 3) & 3], nullptr);
+    pages = pages_of(step + 4);
+    const int tile = kKG * step + kg;
     if (active && tile < tiles) {
       mfma_acc4 s[kRF][4];
-      scores(buf, tile, s);
+      scores(sh.tiles[step & 3], tile, s);
 #pragma unroll
       for (int rf = 0; rf < kRF; ++rf) {
-        float mt = s[rf][0][0];
+        float m_new = m[rf];
 #pragma unroll
         for (int kf = 0; kf < 4; ++kf) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) mt = fmaxf(mt, s[rf][kf][v]);
+          for (int v = 0; v < 4; ++v) m_new = fmaxf(m_new, s[rf][kf][v]);
         }
-        mt = fmaxf(mt, xor_lane<16>(mt));
-        mt = fmaxf(mt, xor_lane<32>(mt));
-        const float m_new = fmaxf(m[rf], mt);
-        // Until a row has seen a visible key in this group (group 1's first
-        // tiles can be fully masked for the early rows) its max is -inf; the
+        // Until a lane has seen a visible key its max is -inf; the
         // exponentials are then taken against 0, all of them are 0, and l
         // stays 0.
         const float neg_base = m_new == -__builtin_huge_valf() ? 0.0f : -m_new * scale_log2e;
@@ -1400,38 +1452,45 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
         m[rf] = m_new;
       }
     }
-    wait_stage_landed<0>();
-    __syncthreads();
   }
-  // Merge the two key groups, group 0 first: M = max(m0, m1),
-  // L = l0 exp(m0 - M) + l1 exp(m1 - M). Group 0 holds key 0, visible to every
-  // row, so M is finite; a group with no visible key has m = -inf and
-  // contributes 0.
+  // Merge a row's four lanes, then the key groups, group 0 first: M = max m,
+  // L = sum of l exp(m - M). Group 0 holds key 0, visible to every row, so M
+  // is finite; lanes and groups with no visible key have m = -inf and
+  // contribute 0.
 #pragma unroll
   for (int rf = 0; rf < kRF; ++rf) {
-    float total = l[rf];
+    float mw = fmaxf(m[rf], xor_lane<16>(m[rf]));
+    mw = fmaxf(mw, xor_lane<32>(mw));
+    float total = mw == -__builtin_huge_valf() ? 0.0f : l[rf] * __builtin_amdgcn_exp2f((m[rf] - mw) * scale_log2e);
     total += xor_lane<16>(total);
     total += xor_lane<32>(total);
     if (grp == 0) {
-      sh.stats[wave][rf * 16 + col][0] = m[rf];
+      sh.stats[wave][rf * 16 + col][0] = mw;
       sh.stats[wave][rf * 16 + col][1] = total;
     }
   }
   __syncthreads();
-  float inv[kRF];
+  // Pass 2's first stage; every wave is past its pass 1 reads.
+  issue(0, pages_of(0), sh.tiles[0], sh.tiles[2]);
+  pages = pages_of(1);
+  float neg_base[kRF];
 #pragma unroll
   for (int rf = 0; rf < kRF; ++rf) {
     const int h = wave & 3;
-    const float m0 = sh.stats[h][rf * 16 + col][0], l0 = sh.stats[h][rf * 16 + col][1];
-    const float m1 = sh.stats[h + 4][rf * 16 + col][0], l1 = sh.stats[h + 4][rf * 16 + col][1];
-    const float M = fmaxf(m0, m1);
-    const float L = __builtin_fmaf(l1, __builtin_amdgcn_exp2f((m1 - M) * scale_log2e),
-                                   l0 * __builtin_amdgcn_exp2f((m0 - M) * scale_log2e));
-    m[rf] = -M * scale_log2e;  // pass 2 takes exp2(c s - c M) as one fma
-    inv[rf] = 1.0f / L;
+    float M = sh.stats[h][rf * 16 + col][0];
+#pragma unroll
+    for (int k = 1; k < kKG; ++k) M = fmaxf(M, sh.stats[h + 4 * k][rf * 16 + col][0]);
+    float L = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kKG; ++k) {
+      L = __builtin_fmaf(sh.stats[h + 4 * k][rf * 16 + col][1],
+                         __builtin_amdgcn_exp2f((sh.stats[h + 4 * k][rf * 16 + col][0] - M) * scale_log2e), L);
+    }
+    // p = exp(s - M) / L as one exponential, exp2(c s - (c M + log2 L)).
+    neg_base[rf] = -__builtin_fmaf(M, scale_log2e, __builtin_amdgcn_logf(L));
   }
 
-  // Pass 2: p = exp(s - M) * (1/L) rounded to the element type, where the
+  // Pass 2: p = exp(s - M) / L rounded to the element type, where the
   // reference rounds its probability buffer, then O^T += V^T . P^T in fp32 per
   // key group; the groups' outputs add at the end, group 0 first.
   mfma_acc4 o[kRF][kDFrags];
@@ -1440,17 +1499,19 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
 #pragma unroll
     for (int df = 0; df < kDFrags; ++df) o[rf][df] = mfma_acc4{0.f, 0.f, 0.f, 0.f};
   }
-  issue(0, 0, true);
-  wait_stage_landed<0>();
-  __syncthreads();
   for (int step = 0; step < steps; ++step) {
     const int buf = step & 1;
-    if (step + 1 < steps) issue(step + 1, buf ^ 1, true);
-    const int tile = kKeyGroups * step + kg;
+    wait_stage_landed<0>();
+    plain_barrier();
+    // buf ^ 1 was last read in the step before
+    if (step + 1 < steps) issue(step + 1, pages, sh.tiles[buf ^ 1], sh.tiles[2 + (buf ^ 1)]);
+    pages = pages_of(step + 2);
+    const int tile = kKG * step + kg;
     if (active && tile < tiles) {
       mfma_acc4 s[kRF][4];
-      scores(buf, tile, s);
-      const elem_t* vt = &sh.values[buf][kg * kFlashKeys * kHeadDim];
+      scores(sh.tiles[buf], tile, s);
+      const elem_t* vt = sh.tiles[2 + buf] + kg * kFlashKeys * kHeadDim;
+      mfma_in8 pb[kRF][2];
 #pragma unroll
       for (int rf = 0; rf < kRF; ++rf) {
         uint32_t pk[4][2];
@@ -1459,42 +1520,47 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
           float pr[4];
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            pr[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[rf][kf][v], scale_log2e, m[rf])) * inv[rf];
+            pr[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[rf][kf][v], scale_log2e, neg_base[rf]));
           }
           pk[kf][0] = pack_rounded(pr[0], pr[1]);
           pk[kf][1] = pack_rounded(pr[2], pr[3]);
         }
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-          const vec16 pw{{pk[2 * half][0], pk[2 * half][1], pk[2 * half + 1][0], pk[2 * half + 1][1]}};
-          const mfma_in8 b = as_operand(pw);
+          pb[rf][half] = as_operand(vec16{{pk[2 * half][0], pk[2 * half][1], pk[2 * half + 1][0], pk[2 * half + 1][1]}});
+        }
+      }
 #pragma unroll
-          for (int df = 0; df < kDFrags; ++df) {
-            o[rf][df] = mfma16x16x32(value_operand(vt, half, df), b, o[rf][df]);
-          }
+      for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int df = 0; df < kDFrags; ++df) {
+          const mfma_in8 va = value_operand(vt, half, df);
+#pragma unroll
+          for (int rf = 0; rf < kRF; ++rf) o[rf][df] = mfma16x16x32(va, pb[rf][half], o[rf][df]);
         }
       }
     }
-    wait_stage_landed<0>();
-    __syncthreads();
   }
 
-  // Group 1 hands its partial output to group 0 through the (now free) key
-  // buffers; group 0 adds it to its own and stores.
-  float* handoff = reinterpret_cast<float*>(&sh.keys[0][0]);
-  static_assert(sizeof(sh.keys) >= 4 * kRF * kDFrags * 4 * 64 * sizeof(float), "handoff must fit");
-  if (kg == 1) {
+  // The other groups hand their partial outputs to group 0 through the (now
+  // free) tile buffers; group 0 adds them to its own in group order and stores.
+  float* handoff = reinterpret_cast<float*>(&sh.tiles[0][0]);
+  constexpr int kHandoff = kRF * kDFrags * 4 * 64;  // floats of a wave
+  static_assert(sizeof(sh.tiles) >= 4 * (kKG - 1) * kHandoff * sizeof(float), "handoff must fit");
+  __syncthreads();
+  if (kg != 0) {
+    float* mine = handoff + (wave - 4) * kHandoff;
 #pragma unroll
     for (int rf = 0; rf < kRF; ++rf) {
 #pragma unroll
       for (int df = 0; df < kDFrags; ++df) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) handoff[((((wave & 3) * kRF + rf) * kDFrags + df) * 4 + v) * 64 + lane] = o[rf][df][v];
+        for (int v = 0; v < 4; ++v) mine[((rf * kDFrags + df) * 4 + v) * 64 + lane] = o[rf][df][v];
       }
     }
   }
   __syncthreads();
-  if (!active || kg == 1) return;
+  if (!active || kg != 0) return;
   // o[rf][df][v] = O[row 16rf + col][dim 16df + 4grp + v]
 #pragma unroll
   for (int rf = 0; rf < kRF; ++rf) {
@@ -1506,7 +1572,13 @@ __global__ __launch_bounds__(kFlashThreads, kHeadDim == 64 ? 4 : 2) void flash_p
     for (int df = 0; df < kDFrags; ++df) {
       float r[4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) r[v] = o[rf][df][v] + handoff[((((wave & 3) * kRF + rf) * kDFrags + df) * 4 + v) * 64 + lane];
+      for (int v = 0; v < 4; ++v) {
+        r[v] = o[rf][df][v];
+#pragma unroll
+        for (int k = 1; k < kKG; ++k) {
+          r[v] += handoff[(wave + 4 * (k - 1)) * kHandoff + ((rf * kDFrags + df) * 4 + v) * 64 + lane];
+        }
+      }
       uint2 packed;
       packed.x = pack_elems(r[0], r[1]);
       packed.y = pack_elems(r[2], r[3]);
@@ -1575,17 +1647,50 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_attention_generic_ker
   if (lane + 64 < head_dim) o[lane + 64] = float_to_elem(acc1);
 }
 
+template <bool kPaged, int kHeadDim, int kRF, int kKG>
+void launch_flash_blocks(elem_t* o, const elem_t* q, const KvCacheView& v, int num_heads, int group,
+                         int tokens, int start_position, float scale_log2e, bool folded, hipStream_t s) {
+  const unsigned zs = static_cast<unsigned>((group + 3) / 4);
+  const int units = (tokens + 16 * kRF - 1) / (16 * kRF) * v.num_kv_heads;
+  const dim3 grid(static_cast<unsigned>((units + 7) / 8 * 8), 1u, zs);
+  flash_prefill_kernel<kPaged, kHeadDim, kRF, kKG><<<grid, 256 * kKG, 0, s>>>(
+      o, q, v, num_heads, group, tokens, start_position, scale_log2e, folded);
+}
+
+// The block for a chunk (T tokens at a start position, 8 kv heads of 4 query
+// heads, 256 compute units; head_dim 64 unless said; each figure against the
+// other blocks' best):
+//  - 32 rows, two key groups, once that still gives every compute unit two
+//    blocks: a tile's LDS reads serve twice the rows. T = 2048: 44.5 us against
+//    47.2 with 16 rows; at start 2048, 102 against 118. At head_dim 128, where
+//    one block fits a compute unit, 75 against 82.
+//  - 16 rows, four key groups (16 waves), where 16-row blocks leave compute
+//    units with one block or none and the keys are many: T = 500 at 6144,
+//    paged, 75 us against 87; T = 200 at 2000 26 against 30. With few keys the
+//    groups find no tiles (T = 77 at 500: 10.4 against 10.2).
+//  - 16 rows, two key groups otherwise (T = 1024: 17.0 us, 22 with 32 rows).
 template <bool kPaged, int kHeadDim>
 void launch_flash(elem_t* o, const elem_t* q, const KvCacheView& v, int num_heads, int group,
                   int tokens, int start_position, float scale, hipStream_t s) {
   const float scale_log2e = static_cast<float>(static_cast<double>(scale) * 1.4426950408889634);
-  const unsigned zs = static_cast<unsigned>((group + 3) / 4);
-  // One row fragment (16 positions) per wave: more, lighter blocks (two per
-  // compute unit) measured faster than two fragments per wave at every T.
-  const int units = (tokens + 15) / 16 * v.num_kv_heads;
-  const dim3 grid(static_cast<unsigned>((units + 7) / 8 * 8), 1u, zs);
-  flash_prefill_kernel<kPaged, kHeadDim, 1><<<grid, kFlashThreads, 0, s>>>(o, q, v, num_heads, group, tokens,
-                                                                          start_position, scale_log2e);
+  const long long cus = device_compute_units();
+  const long long heads = static_cast<long long>(v.num_kv_heads) * ((group + 3) / 4);
+  const long long units32 = (tokens + 31) / 32 * heads;
+  const long long units16 = (tokens + 15) / 16 * heads;
+  if (units32 >= 2 * cus) {
+    const bool folded = kHeadDim == 64 && units32 <= 2 * cus;
+    launch_flash_blocks<kPaged, kHeadDim, 2, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e,
+                                                folded, s);
+    return;
+  }
+  if constexpr (kHeadDim == 64) {
+    if (units16 <= cus && start_position + tokens >= 1024) {
+      launch_flash_blocks<kPaged, kHeadDim, 1, 4>(o, q, v, num_heads, group, tokens, start_position, scale_log2e,
+                                                  false, s);
+      return;
+    }
+  }
+  launch_flash_blocks<kPaged, kHeadDim, 1, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e, false, s);
 }
 
 }  // namespace
