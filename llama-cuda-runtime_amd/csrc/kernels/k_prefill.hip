@@ -696,7 +696,9 @@ constexpr int kRingK = 32;
 //  - 192 x 128, kWaves = 8: wave tiles of 96 x 32 (three 64-row heads per
 //    block tile), so 3072 q/k/v rows and 2048 tokens make exactly 256 tiles;
 //  - 128 x 128, kWaves = 8: wave tiles of 64 x 32, for projections whose
-//    larger tiles would leave compute units idle (two blocks fit a CU).
+//    larger tiles would leave compute units idle (two blocks fit a CU);
+//  - 64 x 128, kWaves = 8: wave tiles of 32 x 32, for few tokens, where the
+//    weights' stream and the split partials count more than the matrix rate.
 // kRK: K per ring stage, 32 (64-byte rows) or 64 (128-byte rows: twice the
 // products per stage barrier). Either way the products run over K in 32-wide
 // MFMA steps in increasing order, so the results are the same bits.
@@ -706,10 +708,11 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
                                                                 GemmGrid grid) {
   static_assert(kRK == 32 || kRK == 64, "ring stages of 32 or 64 K");
   static_assert((BW == 256 && BT == 256 && (kWaves == 4 || kWaves == 8)) ||
-                    ((BW == 256 || BW == 192 || BW == 128) && BT == 128 && kWaves == 8),
-                "supported ring tiles: 256 x 256 on 4 or 8 waves, 256 x 128, 192 x 128 and 128 x 128 on 8 waves");
+                    ((BW == 256 || BW == 192 || BW == 128 || BW == 64) && BT == 128 && kWaves == 8),
+                "supported ring tiles: 256 x 256 on 4 or 8 waves, 256 x 128, 192 x 128, 128 x 128 and 64 x 128 on 8 "
+                "waves");
   // waves along W; the rest split the tokens
-  constexpr int kWavesW = (BW == 128 || BW == 192 || BT == 256) ? 2 : 4;
+  constexpr int kWavesW = (BW <= 192 || BT == 256) ? 2 : 4;
   constexpr int kWavesT = kWaves / kWavesW;
   constexpr int FW = BW / kWavesW / 16;  // W fragments of 16 rows per wave
   constexpr int FT = BT / kWavesT / 16;      // token fragments of 16 tokens per wave
@@ -851,22 +854,29 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
 constexpr int kRingStages = 4;
 // Fraction of a compute unit's MFMA peak the 256 x 128 ring tile reaches
 // (measured on MI355X; the plan compares it with the other shapes').
-constexpr double kRing256x128Efficiency = 0.30;
+constexpr double kRing256x128Efficiency = 0.375;
 // 64 K per stage, three stages (144 KiB of LDS): half the stage barriers of 32
 // K per stage, the same bits; prefill 2.415 -> 2.356 ms at 512 tokens (with
 // the 128 x 128 tile below as well: 2.328 ms, and 6.231 -> 6.115 ms at 2048).
 constexpr int kRing256x128K = 64;
 constexpr int kRing256x128Stages = 3;
 // The 128 x 128 ring tile: o_proj at 2048 tokens (one tile per compute unit)
-// takes 24.2 us, 0.28 of a compute unit's peak, against 34-36 us for the
+// takes 24.2 us, 0.31 of a compute unit's peak past its fill, against 34-36 us for the
 // register-staged 128 x 128 kernel.
-constexpr double kRing128x128Efficiency = 0.28;
+constexpr double kRing128x128Efficiency = 0.31;
 // The 192 x 128 ring tile: three stages of 64 K (120 KiB of LDS).
-constexpr double kRing192x128Efficiency = 0.29;
+constexpr double kRing192x128Efficiency = 0.36;
 constexpr int kRing192x128K = 64;
 constexpr int kRing192x128Stages = 3;
 constexpr int kRing128x128K = 64;  // 64 K per stage, four stages (128 KiB of LDS)
 constexpr int kRing128x128Stages = 4;
+// The 64 x 128 ring tile: three stages of 64 K (72 KiB of LDS, two blocks fit
+// a CU). With 77 tokens, cold weights, against the 128 x 128 tile's best split:
+// down 15.4 us (18.2), q/k/v 11.5 (14.0), o_proj 10.6 (12.2), each with its
+// reduction; four or six stages, or 128 K a stage, measured no faster.
+constexpr double kRing64x128Efficiency = 0.20;
+constexpr int kRing64x128K = 64;
+constexpr int kRing64x128Stages = 3;
 // Waves per ring block. Eight (two per SIMD) measured faster than four with
 // 128 x 128 wave tiles: 143 against 176 us for T = 2048, N = 16384, K = 2048;
 // one wave per SIMD leaves the LDS and barrier latencies uncovered.
@@ -1002,7 +1012,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(void* __restrict__ Y, 
   }
 }
 
-enum class GemmShape { kRing256x256, kRing256x128, kRing192x128, kRing128x128, k256x256, k256x128, k128x128 };
+enum class GemmShape {
+  kRing256x256, kRing256x128, kRing192x128, kRing128x128, kRing64x128, k256x256, k256x128, k128x128
+};
 
 struct GemmPlan {
   GemmShape shape;
@@ -1013,38 +1025,55 @@ struct GemmPlan {
 };
 
 // The plan with the least estimated time. Work units (tile x K slice) run in
-// whole rounds over the compute units; a unit costs its flops at the shape's
-// measured fraction of a compute unit's MFMA peak. Splitting K is considered
-// only when the tiles alone leave compute units idle, and costs the fp32
-// partials' round trip through memory plus a launch. Each slice keeps at
-// least 256 K and is a whole number of the shape's K stages. With
+// whole rounds over the compute units; a plan costs its shape's fill (launch,
+// ring fill, epilogue) and, a round, a unit's flops at the shape's measured
+// fraction of a compute unit's MFMA peak. Splitting K is considered only when
+// the tiles alone leave compute units idle, and costs a reduction: a launch, a
+// part per slice, and the fp32 partials' round trip through memory. A product
+// with N <= K is a projection back onto the residual stream: a residual norm
+// follows, which takes a split's reduction into its own pass, so the unsplit
+// plan pays for that pass (o_proj with its norm, 640 tokens: 128 x 128 in two
+// slices 18.8 us, 64 x 128 unsplit 20.5; q/k/v, where nothing follows, 20.0
+// and 17.9). The plan depends on the sizes alone, not on the entry, so that
+// every fused entry gives the bits of the plain product.
+// Fitted to T = 64 .. 1024 over the four projections of a 2048-wide layer,
+// every tile and split forced in turn (o_proj at 256 tokens: 64 x 128 in four
+// slices 13.9 us, 128 x 128 in four 15.2, in eight 18.5; the estimates order
+// them so; before the fill, slice and norm terms eight was chosen). Each slice
+// keeps at least 256 K and is a whole number of the shape's K stages. With
 // wide_waves, an unsplit plan uses only shapes whose waves own 128 W rows
 // (the RoPE epilogue for 128-row heads). The 192-row tile is for unsplit
-// plans, and without narrow_ok for none (its RoPE epilogue needs the staged
-// store).
+// plans, and without narrow_ok neither it nor the 64-row tile runs unsplit
+// (their RoPE epilogue needs the staged store).
 GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wide_waves = false,
                    bool narrow_ok = true) {
   struct Option {
     GemmShape shape;
     int bw, bt, stage_k;
     double efficiency;  // fraction of a compute unit's MFMA peak, measured on MI355X
+    double fill;        // seconds
   };
   // A ring shape needs K in whole ring stages of its depth.
   const bool ring = K % kRingK == 0;
   const bool ring256x128 = K % kRing256x128K == 0;
   const bool ring128x128 = K % kRing128x128K == 0;
   const bool ring192x128 = K % kRing192x128K == 0;
+  const bool ring64x128 = K % kRing64x128K == 0;
   const Option options[] = {
-      {ring ? GemmShape::kRing256x256 : GemmShape::k256x256, 256, 256, ring ? kRingK : kStageK, ring ? 0.37 : 0.31},
+      {ring ? GemmShape::kRing256x256 : GemmShape::k256x256, 256, 256, ring ? kRingK : kStageK, ring ? 0.415 : 0.31,
+       4e-6},
       {ring256x128 ? GemmShape::kRing256x128 : GemmShape::k256x128, 256, 128,
-       ring256x128 ? kRing256x128K : kStageK, ring256x128 ? kRing256x128Efficiency : 0.23},
+       ring256x128 ? kRing256x128K : kStageK, ring256x128 ? kRing256x128Efficiency : 0.23, 3e-6},
       {ring128x128 ? GemmShape::kRing128x128 : GemmShape::k128x128, 128, 128,
-       ring128x128 ? kRing128x128K : kStageK, ring128x128 ? kRing128x128Efficiency : 0.20},
-      // ring only: the register-staged kernel has no 192-row tile
-      {GemmShape::kRing192x128, 192, 128, kRing192x128K, ring192x128 ? kRing192x128Efficiency : 0.0}};
+       ring128x128 ? kRing128x128K : kStageK, ring128x128 ? kRing128x128Efficiency : 0.20, 3e-6},
+      // ring only: the register-staged kernel has no 192- or 64-row tile
+      {GemmShape::kRing192x128, 192, 128, kRing192x128K, ring192x128 ? kRing192x128Efficiency : 0.0, 3e-6},
+      {GemmShape::kRing64x128, 64, 128, kRing64x128K, ring64x128 ? kRing64x128Efficiency : 0.0, 2e-6}};
   constexpr double kCuPeak = 9.8e12;     // bf16 dense flop/s per compute unit
-  constexpr double kBandwidth = 5.0e12;  // sustained bytes/s for the partials' round trip
-  constexpr double kLaunch = 4e-6;
+  constexpr double kBandwidth = 5.0e12;  // sustained bytes/s for the partials' round trip, the norm's rows
+  constexpr double kReduce = 3e-6;
+  constexpr double kSlice = 0.5e-6;
+  constexpr double kNorm = 1.5e-6;
   GemmPlan best{GemmShape::k128x128, 128, 128, 1, K, 0};
   double best_time = -1.0;
   for (const Option& o : options) {
@@ -1059,11 +1088,17 @@ GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wi
       // 192-row tiles unsplit only: split four ways for q/k/v at 512 tokens
       // they measured slower than 128 x 128 tiles split in two
       if (o.bw == 192 && (used > 1 || !narrow_ok)) continue;
+      if (o.bw == 64 && used == 1 && !narrow_ok) continue;
       const size_t bytes = used > 1 ? static_cast<size_t>(used) * T * N * sizeof(float) : 0;
       if (bytes > workspace_bytes) break;
       const long long rounds = (tiles * used + cus - 1) / cus;
-      double time = static_cast<double>(rounds) * 2.0 * o.bw * o.bt * k_chunk / (o.efficiency * kCuPeak);
-      if (used > 1) time += (static_cast<double>(bytes) + static_cast<double>(T) * N * 4.0) / kBandwidth + kLaunch;
+      double time =
+          o.fill + static_cast<double>(rounds) * 2.0 * o.bw * o.bt * k_chunk / (o.efficiency * kCuPeak);
+      if (used > 1) {
+        time += kReduce + used * kSlice + static_cast<double>(bytes) / kBandwidth;
+      } else if (N <= K) {
+        time += kNorm + static_cast<double>(T) * N * 4.0 / kBandwidth;
+      }
       if (best_time < 0.0 || time < best_time) {
         best = GemmPlan{o.shape, o.bw, o.bt, used, k_chunk, bytes};
         best_time = time;
@@ -1128,6 +1163,9 @@ bool run_gemm(void* Y, bool fp32_out, const elem_t* X, const elem_t* W, int T, i
       break;
     case GemmShape::kRing192x128:
       launch_gemm_ring<192, 128, 8, kRing192x128Stages, kRing192x128K>(Y, fp32_out, X, W, T, N, K, grid, s);
+      break;
+    case GemmShape::kRing64x128:
+      launch_gemm_ring<64, 128, 8, kRing64x128Stages, kRing64x128K>(Y, fp32_out, X, W, T, N, K, grid, s);
       break;
     case GemmShape::k256x256:
       launch_gemm_tiles<256, 256, 2, 4>(Y, fp32_out, X, W, T, N, K, grid, s);
