@@ -29,6 +29,7 @@
 // it to the element type (the reference's probability buffer) and accumulates
 // p * v in fp32, rounded once on store.
 #include <algorithm>
+#include <type_traits>
 
 #include "../capi_util.h"
 #include "../kv_cache.h"
@@ -753,12 +754,13 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
                            : X + static_cast<size_t>(min(t0 + row - BW, T - 1)) * K) + work.k_first + 8 * chunk;
   }
   const uint32_t ring_base = lds_address_of(ring) + static_cast<uint32_t>(wave * 1024);
-  auto issue = [&](int s) {
+  auto issue_load = [&](int s, int i) {
     const uint32_t base = ring_base + static_cast<uint32_t>((s % kStages) * kStageElems * 2);
+    load_to_lds16(src[i] + s * kRK, base + static_cast<uint32_t>(i * kWaves * 1024));
+  };
+  auto issue = [&](int s) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      load_to_lds16(src[i] + s * kRK, base + static_cast<uint32_t>(i * kWaves * 1024));
-    }
+    for (int i = 0; i < kLoads; ++i) issue_load(s, i);
   };
 
   mfma_acc4 acc[FW][FT];
@@ -785,10 +787,22 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
 #pragma unroll
     for (int j = 0; j < FT; ++j) bt[j] = lds_operand(base + (BW + wt + 16 * j + col) * kRK);
   };
-  // Products of the stage whose fragments are in aw / bt, reading stage
-  // `next` into aw / bt_next. After the last stage `next` repeats a stage
-  // whose loads have all landed, and what is read goes unused.
-  auto step = [&](const mfma_in8 (&bt)[FT], mfma_in8 (&bt_next)[FT], int next) {
+  // Products of the k-step whose fragments are in aw / bt, reading k-step
+  // `next` into aw / bt_next. After the last k-step `next` repeats one whose
+  // loads have all landed, and what is read goes unused.
+  // kPart >= 0: this is k-step kPart of the kKSteps that share the loads of
+  // stage `fill`; a load follows the products of each W fragment, until the
+  // stage's are spent. A compute unit takes a 1 KB load every 16 cycles or so,
+  // and all its waves leave the stage barrier together: issued there in one
+  // burst, the loads hold every wave off its products for that long (without
+  // any loads gate/up at 512 tokens ran 29.5 us instead of 41.5, with every
+  // load from one hot address still 40.5). Spread over the products, bursts at
+  // the barrier against now: gate/up 41.5 -> 37.6 us, down 30.5 -> 26.8, q/k/v
+  // 17.8 -> 14.0, o_proj 17.1 -> 15.5 (512 tokens); 135.5 -> 133.2, 75.0 ->
+  // 71.1, 30.2 -> 25.2, 28.7 -> 25.6 (2048).
+  constexpr int kSlots = FW * kKSteps;
+  auto step = [&](const mfma_in8 (&bt)[FT], mfma_in8 (&bt_next)[FT], int next, auto part, int fill) {
+    constexpr int kPart = decltype(part)::value;
     const elem_t* nb =
         ring + ((next / kKSteps) % kStages) * kStageElems + (ww + col) * kRK + swz(next % kKSteps);
     read_tokens(next, bt_next);
@@ -802,20 +816,30 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
 #pragma unroll
       for (int j = 0; j < FT; ++j) acc[i][j] = mfma16x16x32(aw[i], bt[j], acc[i][j]);
       aw[i] = lds_operand(nb + 16 * i * kRK);
-    }
-    // keep that order: the token reads, then per W fragment its products and
-    // its replacement's read
-    __builtin_amdgcn_sched_group_barrier(0x100, FT, 0);
+      if constexpr (kPart >= 0) {
 #pragma unroll
-    for (int i = 0; i < FW; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, FT, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        for (int l = 0; l < kLoads; ++l) {
+          if (l * kSlots / kLoads == kPart * FW + i) issue_load(fill, l);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (kPart < 0) {
+      // keep that order: the token reads, then per W fragment its products and
+      // its replacement's read
+      __builtin_amdgcn_sched_group_barrier(0x100, FT, 0);
+#pragma unroll
+      for (int i = 0; i < FW; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, FT, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
     }
     __builtin_amdgcn_s_setprio(0);
   };
   // Before reading stage `next`: this wave's loads of it have landed (at most
   // the loads of the stages issued after it remain) and its earlier fragment
-  // reads have returned; then the block meets and the freed buffer is refilled.
+  // reads have returned; then the block meets, and the buffer of the stage
+  // before it is free for stage next + kStages - 1.
   auto advance = [&](int next) {
     if (next + kStages - 2 < stages) {
       wait_stage_landed<kLoads * (kStages - 2)>();
@@ -823,23 +847,41 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
       wait_stage_landed<0>();
     }
     __builtin_amdgcn_s_barrier();
-    if (next + kStages - 1 < stages) issue(next + kStages - 1);
   };
   for (int s = 0; s < kStages - 1 && s < stages; ++s) issue(s);
   advance(0);
+  if (kStages - 1 < stages) issue(kStages - 1);
   read_tokens(0, bt_a);
   {
     const elem_t* base = ring + (ww + col) * kRK + swz(0);
 #pragma unroll
     for (int i = 0; i < FW; ++i) aw[i] = lds_operand(base + 16 * i * kRK);
   }
-  for (int q = 0; q < ksteps; ++q) {
-    // Reading k-step q + 1's fragments opens a new stage every kKSteps steps.
-    if (q + 1 < ksteps && (q + 1) % kKSteps == 0) advance((q + 1) / kKSteps);
-    step(bt_a, bt_b, min(q + 1, ksteps - 1));
+  auto run_step = [&](int q, auto part, int fill) {
+    step(bt_a, bt_b, min(q + 1, ksteps - 1), part, fill);
 #pragma unroll
     for (int j = 0; j < FT; ++j) bt_a[j] = bt_b[j];
+  };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
+  using NoLoads = std::integral_constant<int, -1>;
+  // K-step q reads q + 1's fragments, so stage `next` opens before its first
+  // k-step's predecessor; the stage behind it in the ring is loaded during
+  // that k-step and the rest of the kKSteps up to the next opening.
+  int q = 0;
+  for (; q < kKSteps - 1; ++q) run_step(q, NoLoads{}, 0);
+  int next = 1;
+  for (; next + kStages - 1 < stages; ++next) {
+    advance(next);
+    run_step(q++, First{}, next + kStages - 1);
+    if constexpr (kKSteps == 2) run_step(q++, Second{}, next + kStages - 1);
   }
+  for (; next < stages; ++next) {
+    advance(next);
+#pragma unroll
+    for (int e = 0; e < kKSteps; ++e) run_step(q++, NoLoads{}, 0);
+  }
+  run_step(q, NoLoads{}, 0);
 
   float* partial = grid.partial != nullptr ? grid.partial + static_cast<size_t>(work.split) * T * N : nullptr;
   if (staged_store_ok(grid, Y, partial, kFp32Out, N)) {
@@ -1039,7 +1081,9 @@ struct GemmPlan {
 // Fitted to T = 64 .. 1024 over the four projections of a 2048-wide layer,
 // every tile and split forced in turn (o_proj at 256 tokens: 64 x 128 in four
 // slices 13.9 us, 128 x 128 in four 15.2, in eight 18.5; the estimates order
-// them so; before the fill, slice and norm terms eight was chosen). Each slice
+// them so; before the fill, slice and norm terms eight was chosen). These times
+// are from before the loads were spread over the products, which made every
+// ring tile faster by 2 to 20 %. Each slice
 // keeps at least 256 K and is a whole number of the shape's K stages. With
 // wide_waves, an unsplit plan uses only shapes whose waves own 128 W rows
 // (the RoPE epilogue for 128-row heads). The 192-row tile is for unsplit
