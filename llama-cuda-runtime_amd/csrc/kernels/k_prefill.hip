@@ -1071,17 +1071,13 @@ struct GemmPlan {
 // ring fill, epilogue) and, a round, a unit's flops at the shape's measured
 // fraction of a compute unit's MFMA peak. Splitting K is considered only when
 // the tiles alone leave compute units idle, and costs a reduction: a launch, a
-// part per slice, and the fp32 partials' round trip through memory. A product
-// with N <= K is a projection back onto the residual stream: a residual norm
-// follows, which takes a split's reduction into its own pass, so the unsplit
-// plan pays for that pass (o_proj with its norm, 640 tokens: 128 x 128 in two
-// slices 18.8 us, 64 x 128 unsplit 20.5; q/k/v, where nothing follows, 20.0
-// and 17.9). The plan depends on the sizes alone, not on the entry, so that
-// every fused entry gives the bits of the plain product.
+// part per slice, and the fp32 partials' round trip through memory. The plan
+// depends on the sizes alone, not on the entry, so that every fused entry gives
+// the bits of the plain product.
 // Fitted to T = 64 .. 1024 over the four projections of a 2048-wide layer,
 // every tile and split forced in turn (o_proj at 256 tokens: 64 x 128 in four
 // slices 13.9 us, 128 x 128 in four 15.2, in eight 18.5; the estimates order
-// them so; before the fill, slice and norm terms eight was chosen). These times
+// them so; before the fill and slice terms eight was chosen). These times
 // are from before the loads were spread over the products, which made every
 // ring tile faster by 2 to 20 %. Each slice
 // keeps at least 256 K and is a whole number of the shape's K stages. With
@@ -1114,10 +1110,9 @@ GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wi
       {GemmShape::kRing192x128, 192, 128, kRing192x128K, ring192x128 ? kRing192x128Efficiency : 0.0, 3e-6},
       {GemmShape::kRing64x128, 64, 128, kRing64x128K, ring64x128 ? kRing64x128Efficiency : 0.0, 2e-6}};
   constexpr double kCuPeak = 9.8e12;     // bf16 dense flop/s per compute unit
-  constexpr double kBandwidth = 5.0e12;  // sustained bytes/s for the partials' round trip, the norm's rows
+  constexpr double kBandwidth = 5.0e12;  // sustained bytes/s for the partials' round trip
   constexpr double kReduce = 3e-6;
   constexpr double kSlice = 0.5e-6;
-  constexpr double kNorm = 1.5e-6;
   GemmPlan best{GemmShape::k128x128, 128, 128, 1, K, 0};
   double best_time = -1.0;
   for (const Option& o : options) {
@@ -1132,17 +1127,16 @@ GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wi
       // 192-row tiles unsplit only: split four ways for q/k/v at 512 tokens
       // they measured slower than 128 x 128 tiles split in two
       if (o.bw == 192 && (used > 1 || !narrow_ok)) continue;
-      if (o.bw == 64 && used == 1 && !narrow_ok) continue;
+      // 64-row tiles unsplit only once they fill the device: short of that
+      // o_proj with its norm at 640 tokens took 20.5 us, against 18.8 with
+      // 128 x 128 tiles split in two
+      if (o.bw == 64 && used == 1 && (!narrow_ok || tiles < cus)) continue;
       const size_t bytes = used > 1 ? static_cast<size_t>(used) * T * N * sizeof(float) : 0;
       if (bytes > workspace_bytes) break;
       const long long rounds = (tiles * used + cus - 1) / cus;
       double time =
           o.fill + static_cast<double>(rounds) * 2.0 * o.bw * o.bt * k_chunk / (o.efficiency * kCuPeak);
-      if (used > 1) {
-        time += kReduce + used * kSlice + static_cast<double>(bytes) / kBandwidth;
-      } else if (N <= K) {
-        time += kNorm + static_cast<double>(T) * N * 4.0 / kBandwidth;
-      }
+      if (used > 1) time += kReduce + used * kSlice + static_cast<double>(bytes) / kBandwidth;
       if (best_time < 0.0 || time < best_time) {
         best = GemmPlan{o.shape, o.bw, o.bt, used, k_chunk, bytes};
         best_time = time;

@@ -66,15 +66,18 @@ def test_narrow_tile_products(gpu, lcr, kind, variant, T, N, K):
         expect_bits_equal(host(x_got), host(x_want), "residual")
 
 
-@pytest.mark.parametrize("T,start,paged,shift", [(64, 0, False, 0), (65, 5, True, 0), (128, 100, True, 0),
-                                                 (500, 3, True, 0), (500, 0, False, 0), (513, 9, True, 0),
-                                                 # caches 8 bytes past a 16-byte boundary: no narrow tile unsplit
-                                                 (500, 3, False, 4), (65, 3, True, 4)])
-def test_narrow_tile_qkv_rope(gpu, lcr, T, start, paged, shift):
-    """3072 q/k/v rows: split in the reduction at few tokens, rotated in the
-    64 x 128 tile's epilogue (one head a tile) at 500."""
+@pytest.mark.parametrize("T,nh,K,start,paged,shift", [
+    # 3072 rows, split: rotated in the reduction
+    (64, 32, 2048, 0, False, 0), (65, 32, 2048, 5, True, 0), (128, 32, 2048, 100, True, 0), (500, 32, 2048, 3, True, 0),
+    # 16384 rows, 256 tiles of one head each: rotated in the tile's epilogue
+    (64, 240, 256, 0, False, 0), (65, 240, 256, 5, True, 0), (128, 240, 320, 100, True, 0),
+    # caches 8 bytes past a 16-byte boundary: no narrow tile unsplit
+    (65, 32, 2048, 3, True, 4), (128, 240, 256, 3, False, 4)])
+def test_narrow_tile_qkv_rope(gpu, lcr, T, nh, K, start, paged, shift):
+    """The q/k/v projection with RoPE and the cache append against the plain
+    product, the RoPE of its queries and the append."""
     lib = lcr.load_library("bf16")
-    nh, kv, hd, K = 32, 8, 64, 2048
+    kv, hd = 8, 64
     N = (nh + 2 * kv) * hd
     r = rng(T + start + shift)
     Xd, Wd = dev(random_elems(r, (T, K))), dev(random_elems(r, (N, K), 0.05))
