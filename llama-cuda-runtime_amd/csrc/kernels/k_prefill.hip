@@ -797,8 +797,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
   // burst, the loads hold every wave off its products for that long (without
   // any loads gate/up at 512 tokens ran 29.5 us instead of 41.5, with every
   // load from one hot address still 40.5). Spread over the products, bursts at
-  // the barrier against now: gate/up 41.5 -> 37.6 us, down 30.5 -> 26.8, q/k/v
-  // 17.8 -> 14.0, o_proj 17.1 -> 15.5 (512 tokens); 135.5 -> 133.2, 75.0 ->
+  // the barrier against now: gate/up 41.5 -> 37.6 us, down 30.5 -> 26.8, 3072
+  // rows in 64 x 128 tiles 17.8 -> 14.0, o_proj 17.1 -> 15.5 (512 tokens); 135.5 -> 133.2, 75.0 ->
   // 71.1, 30.2 -> 25.2, 28.7 -> 25.6 (2048).
   constexpr int kSlots = FW * kKSteps;
   auto step = [&](const mfma_in8 (&bt)[FT], mfma_in8 (&bt_next)[FT], int next, auto part, int fill) {
@@ -903,8 +903,8 @@ constexpr double kRing256x128Efficiency = 0.375;
 constexpr int kRing256x128K = 64;
 constexpr int kRing256x128Stages = 3;
 // The 128 x 128 ring tile: o_proj at 2048 tokens (one tile per compute unit)
-// takes 24.2 us, 0.31 of a compute unit's peak past its fill, against 34-36 us for the
-// register-staged 128 x 128 kernel.
+// took 24.2 us, 0.31 of a compute unit's peak past its fill, against 34-36 us
+// for the register-staged 128 x 128 kernel.
 constexpr double kRing128x128Efficiency = 0.31;
 // The 192 x 128 ring tile: three stages of 64 K (120 KiB of LDS).
 constexpr double kRing192x128Efficiency = 0.36;
