@@ -846,7 +846,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
     } else {
       wait_stage_landed<0>();
     }
-    __builtin_amdgcn_s_barrier();
+    plain_barrier();
   };
   for (int s = 0; s < kStages - 1 && s < stages; ++s) issue(s);
   advance(0);

@@ -43,6 +43,18 @@ def test_library_exports_every_declared_symbol(lcr, variant):
     assert set(names) <= set(lcr.SIGNATURES), sorted(set(names) - set(lcr.SIGNATURES))
 
 
+def test_block_barriers_fence_memory():
+    """Kernels that wait for their loads by hand meet at plain_barrier(), which
+    keeps the compiler from moving a shared-memory access across it; the bare
+    builtin is no fence for loads issued from inline assembly."""
+    kernels = REPO / "llama-cuda-runtime_amd" / "csrc" / "kernels"
+    bare = [f"{path.name}:{i}" for path in sorted(kernels.iterdir())
+            for i, line in enumerate(path.read_text().splitlines(), 1)
+            if "__builtin_amdgcn_s_barrier" in line.split("//")[0]]
+    (definition,) = [b for b in bare if b.startswith("device_common.h:")]
+    assert bare == [definition]
+
+
 def test_elem_names(lcr):
     assert lcr.load_library("bf16").lcr_elem_name() == b"bf16"
     assert lcr.load_library("fp16").lcr_elem_name() == b"fp16"
