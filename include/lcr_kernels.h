@@ -202,8 +202,8 @@ int lcr_rope_table(float* table, const float* inv_freq, int positions, int head_
 
 /* The fused q/k/v projection of src/model.cu:393 followed by launch_rope_q and
  * launch_rope_write_kv (src/model.cu:396-406, src/kernels.cuh:62-72) in one
- * pass, bit-identical to lcr_gemm_ws into a [T][N] buffer and those two
- * kernels reading it: each output is rounded to the element type, queries
+ * pass, bit-identical to lcr_gemm_ws (with the same workspace) into a [T][N]
+ * buffer and those two kernels reading it: each output is rounded to the element type, queries
  * are rotated into q_heads [num_heads][T][head_dim], keys rotated and values
  * copied into the cache through the view at positions start_position + t.
  * W_qkv holds the num_heads query heads, then the view's num_kv_heads key and

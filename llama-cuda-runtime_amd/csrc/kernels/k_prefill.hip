@@ -119,10 +119,13 @@ constexpr int kGemmPitch = kStageK;
 // rounded to the element type, as a 16-bit GEMM output would be; queries are
 // then rotated into q_heads [num_heads][T][head_dim], keys rotated and values
 // copied into the cache at position start_position + t, with the arithmetic
-// of the separate RoPE kernels reading a 16-bit output. The unsplit epilogue
-// pairs element i of a head with i + head_dim / 2 inside one lane (fragments
-// m and m + head_dim / 32 of a 64- or 128-row head block), so a wave's rows
-// must hold whole heads; split launches rotate in the reduction.
+// of the separate RoPE kernels reading a 16-bit output. Unsplit launches rotate
+// in the epilogue, whose unit is 64 logical rows (RopePiece): 32 elements of a
+// head, then the 32 they pair with. A 64-row head is one such piece as it
+// stands; of a 128-row head, piece h (0 or 1) holds rows 32 h .. + 31 and
+// 64 + 32 h .. + 31 (weight_row). Every tile's rows are whole pieces, so the
+// tile is chosen without regard to the head size. Split launches keep the
+// weight's row order and rotate in the reduction.
 struct GemmRope {
   const float2* table;  // (cos, sin) of position p, pair i at p * head_dim / 2 + i
   elem_t* q_heads;
@@ -139,11 +142,18 @@ struct GemmGrid {
   int k_chunk;
   float* partial;  // nullptr: no split, write Y
   int ffn;         // > 0: gated (Y is act[T][ffn], N == 2 * ffn)
+  int half_heads;  // rows in the pieces of 128-row heads (unsplit RoPE launches)
+  // RoPE: the cache's rows lie on 8-byte boundaries only. Here and not behind
+  // `rope`, whose arguments arrive later: read there by the epilogue, 2048 tokens
+  // of 3072 rows took 0.4 us longer.
+  int narrow_cache;
   GemmRope rope;
 };
 
-__device__ __forceinline__ int weight_row(int p, int ffn) {
-  return ffn == 0 ? p : (((p >> 5) << 4) | (p & 15)) + ((p & 16) ? ffn : 0);
+__device__ __forceinline__ int weight_row(int p, const GemmGrid& g) {
+  if (g.ffn > 0) return (((p >> 5) << 4) | (p & 15)) + ((p & 16) ? g.ffn : 0);
+  if (g.half_heads) return (p & ~127) + ((p & 64) >> 1) + (p & 31) + ((p & 32) << 1);
+  return p;
 }
 
 __device__ __forceinline__ float swiglu_rounded(float gate, float up) {
@@ -190,55 +200,41 @@ __device__ __forceinline__ void emit_rope_quad(const GemmRope& r, int T, int t, 
   *reinterpret_cast<uint2*>(dst + half) = uint2{pack_elems(b[0], b[1]), pack_elems(b[2], b[3])};
 }
 
-// The unsplit RoPE epilogue for heads of 32 kHalfFrags rows: fragment m of a
-// head block holds pairs 16 m + 4 grp + v, its partner fragment m + kHalfFrags
-// the matching high halves.
-template <int FW, int FT, int kHalfFrags, bool kPaged>
+// Where 64 logical rows from `row` on belong: the head's first projection row
+// and the first of the 32 pairs.
+struct RopePiece {
+  int row0, i0;
+};
+__device__ __forceinline__ RopePiece rope_piece(int row, int head_dim) {
+  return head_dim == 64 ? RopePiece{row, 0} : RopePiece{row & ~127, (row & 64) >> 1};
+}
+
+// The unsplit RoPE epilogue from registers: fragments 4 k + m of a wave's rows
+// hold pairs 16 m + 4 grp + v (m < 2) of its piece k, fragments 4 k + 2 + m the
+// matching high halves.
+template <int FW, int FT, bool kPaged>
 __device__ __forceinline__ void store_rope_tile(const mfma_acc4 (&acc)[FW][FT], const GemmRope& r, int T, int N,
                                                 int t_base, int w_base, int col, int grp) {
-  constexpr int kHeadDim = 32 * kHalfFrags;
-  static_assert(FW % (2 * kHalfFrags) == 0, "a wave's rows hold whole heads");
+  static_assert(FW % 4 == 0, "a wave's rows are whole pieces");
+  const int head_dim = r.view.head_dim;
 #pragma unroll
   for (int j = 0; j < FT; ++j) {
     const int t = t_base + j * 16 + col;
     if (t >= T) continue;
 #pragma unroll
-    for (int hb = 0; hb < FW / (2 * kHalfFrags); ++hb) {
-      const int row0 = w_base + hb * kHeadDim;
-      if (row0 >= N) continue;
+    for (int k = 0; k < FW / 4; ++k) {
+      if (w_base + 64 * k >= N) continue;
+      const RopePiece piece = rope_piece(w_base + 64 * k, head_dim);
 #pragma unroll
-      for (int m = 0; m < kHalfFrags; ++m) {
-        const int f = 2 * kHalfFrags * hb + m;
+      for (int m = 0; m < 2; ++m) {
         float lo[4], hi[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          lo[v] = round_to_elem(acc[f][j][v]);
-          hi[v] = round_to_elem(acc[f + kHalfFrags][j][v]);
+          lo[v] = round_to_elem(acc[4 * k + m][j][v]);
+          hi[v] = round_to_elem(acc[4 * k + 2 + m][j][v]);
         }
-        emit_rope_quad<kPaged>(r, T, t, row0, 16 * m + 4 * grp, kHeadDim, lo, hi);
+        emit_rope_quad<kPaged>(r, T, t, piece.row0, piece.i0 + 16 * m + 4 * grp, head_dim, lo, hi);
       }
-    }
-  }
-}
-
-template <int FW, int FT>
-__device__ __forceinline__ void store_rope_heads(const mfma_acc4 (&acc)[FW][FT], const GemmRope& r, int T, int N,
-                                                 int t_base, int w_base, int col, int grp) {
-  // Waves whose rows are not whole heads (the 192-row tile) always take the
-  // staged epilogue; the planner gives them no other case.
-  if (r.view.head_dim == 64) {
-    if constexpr (FW % 4 == 0) {
-      if (r.paged) {
-        store_rope_tile<FW, FT, 2, true>(acc, r, T, N, t_base, w_base, col, grp);
-      } else {
-        store_rope_tile<FW, FT, 2, false>(acc, r, T, N, t_base, w_base, col, grp);
-      }
-    }
-  } else if constexpr (FW % 8 == 0) {
-    if (r.paged) {
-      store_rope_tile<FW, FT, 4, true>(acc, r, T, N, t_base, w_base, col, grp);
-    } else {
-      store_rope_tile<FW, FT, 4, false>(acc, r, T, N, t_base, w_base, col, grp);
     }
   }
 }
@@ -270,12 +266,6 @@ __device__ __forceinline__ void store_gemm_tile(const mfma_acc4 (&acc)[FW][FT], 
                                                 int T, int N, int t_base, int w_base, int col, int grp,
                                                 const GemmGrid& grid) {
   const int ffn = grid.ffn;
-  if constexpr (!kFp32Out) {
-    if (grid.rope.table != nullptr && partial == nullptr) {
-      store_rope_heads<FW, FT>(acc, grid.rope, T, N, t_base, w_base, col, grp);
-      return;
-    }
-  }
   if (ffn > 0 && partial == nullptr) {
     // fragments 2m (gate) and 2m + 1 (up): features (w_base + 32m) / 2 + 4grp + v
 #pragma unroll
@@ -370,15 +360,13 @@ struct StagedTile {
 };
 
 // Whether the ring kernel's epilogue goes through StagedTile: when every
-// destination is 16-byte aligned and its rows are whole 16-byte chunks.
+// destination is 16-byte aligned and its rows are whole 16-byte chunks. The
+// RoPE epilogue always does: queries are aligned, and cache rows that are not
+// take 8-byte stores.
 __device__ __forceinline__ bool staged_store_ok(const GemmGrid& grid, const void* Y, const float* partial,
                                                 bool fp32_out, int N) {
   if (partial == nullptr && !fp32_out && grid.rope.table != nullptr) {
-    // The RoPE epilogue writes 16-byte chunks of query rows and cache rows.
-    const KvCacheView& v = grid.rope.view;
-    return ((reinterpret_cast<uintptr_t>(grid.rope.q_heads) | reinterpret_cast<uintptr_t>(v.keys) |
-             reinterpret_cast<uintptr_t>(v.values)) & 15) == 0 &&
-           (v.page_stride & 7) == 0 && (v.head_stride & 7) == 0;
+    return true;
   }
   const void* out = partial != nullptr ? static_cast<const void*>(partial) : Y;
   if ((reinterpret_cast<uintptr_t>(out) & 15) != 0) return false;
@@ -388,64 +376,91 @@ __device__ __forceinline__ bool staged_store_ok(const GemmGrid& grid, const void
 
 // The RoPE epilogue from a staged tile of 16-bit projection outputs (already
 // rounded, as the unfused path rounds the q/k/v buffer): thread item (token
-// row, group of eight pairs i .. i + 7) loads that position's eight (cos, sin)
-// once and serves every head of the tile with them, rotating a query or key
-// head's pairs (i, i + half) into q_heads or the keys, or copying a value
-// head's; each write is a 16-byte chunk. The same arithmetic as
+// row, group of eight pairs i .. i + 7 of a piece) loads that position's eight
+// (cos, sin) once (once per half of 128-row heads) and serves every piece of the
+// tile with them, rotating query or key pairs (i, i + half) into q_heads or the
+// keys, or copying values; each write is a 16-byte chunk. The same arithmetic as
 // emit_rope_quad, so the same bits.
 template <int kHd, bool kPaged, int BW, int BT, int kThreads, class Tile>
 __device__ __forceinline__ void rope_copy_out(const Tile& tile, const GemmRope& r, int T, int N, int t0, int w0) {
   constexpr int kHalf = kHd / 2;
-  constexpr int kGroups = kHalf / 8;
-  constexpr int kHeads = BW / kHd;
-  constexpr int kItems = BT * kGroups;
-  static_assert(BW % kHd == 0 && kItems % kThreads == 0, "whole heads per tile, whole item rounds");
+  constexpr int kPieces = BW / 64;
+  constexpr int kParts = kHd / 64;  // pieces of a head
+  constexpr int kItems = BT * 4;
+  static_assert(BW % 64 == 0 && kItems % kThreads == 0, "whole pieces per tile, whole item rounds");
   const int kv_dim = r.view.num_kv_heads * kHd;
 #pragma unroll
   for (int it = 0; it < kItems / kThreads; ++it) {
     const int item = it * kThreads + static_cast<int>(threadIdx.x);
-    const int row = item / kGroups;
-    const int i = 8 * (item % kGroups);
+    const int row = item / 4;
     const int t = t0 + row;
     if (t >= T) continue;
     const int position = r.start_position + t;
-    const float4* cs4 = reinterpret_cast<const float4*>(r.table + static_cast<size_t>(position) * kHalf + i);
-    float2 c[8];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 w = cs4[q];
-      c[2 * q] = make_float2(w.x, w.y);
-      c[2 * q + 1] = make_float2(w.z, w.w);
-    }
+    for (int part = 0; part < kParts; ++part) {
+      const int first = kParts == 1 ? 0 : ((w0 >> 6) + part) & 1;  // the tile's first piece of this part
+      if (first >= kPieces) continue;
+      const int i = 32 * part + 8 * (item % 4);
+      const float4* cs4 = reinterpret_cast<const float4*>(r.table + static_cast<size_t>(position) * kHalf + i);
+      float2 c[8];
 #pragma unroll
-    for (int hb = 0; hb < kHeads; ++hb) {
-      const int row0 = w0 + hb * kHd;
-      if (row0 >= N) break;
-      const vec16 lo_v = *reinterpret_cast<const vec16*>(tile.slot(row, (hb * kHd + i) * 2));
-      const vec16 hi_v = *reinterpret_cast<const vec16*>(tile.slot(row, (hb * kHd + kHalf + i) * 2));
-      if (row0 >= r.q_dim + kv_dim) {
-        elem_t* dst = r.view.values + r.view.offset<kPaged>((row0 - r.q_dim - kv_dim) / kHd, position) + i;
-        store16(dst, lo_v);
-        store16(dst + kHalf, hi_v);
-        continue;
+      for (int q = 0; q < 4; ++q) {
+        const float4 w = cs4[q];
+        c[2 * q] = make_float2(w.x, w.y);
+        c[2 * q + 1] = make_float2(w.z, w.w);
       }
-      float lo[8], hi[8];
-      unpack8(lo_v, lo);
-      unpack8(hi_v, hi);
-      vec16 a, b;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float2 r0 = rope_rotate(lo[2 * v], hi[2 * v], c[2 * v]);
-        const float2 r1 = rope_rotate(lo[2 * v + 1], hi[2 * v + 1], c[2 * v + 1]);
-        a.w[v] = pack_elems(r0.x, r1.x);
-        b.w[v] = pack_elems(r0.y, r1.y);
+      for (int n = 0; n < (kPieces + kParts - 1) / kParts; ++n) {
+        const int k = first + kParts * n;
+        if (k >= kPieces || w0 + 64 * k >= N) break;
+        const int row0 = rope_piece(w0 + 64 * k, kHd).row0;
+        const int byte = (64 * k + 8 * (item % 4)) * 2;
+        const vec16 lo_v = *reinterpret_cast<const vec16*>(tile.slot(row, byte));
+        const vec16 hi_v = *reinterpret_cast<const vec16*>(tile.slot(row, byte + 64));
+        if (row0 >= r.q_dim + kv_dim) {
+          elem_t* dst = r.view.values + r.view.offset<kPaged>((row0 - r.q_dim - kv_dim) / kHd, position) + i;
+          store16(dst, lo_v);
+          store16(dst + kHalf, hi_v);
+          continue;
+        }
+        float lo[8], hi[8];
+        unpack8(lo_v, lo);
+        unpack8(hi_v, hi);
+        vec16 a, b;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float2 r0 = rope_rotate(lo[2 * v], hi[2 * v], c[2 * v]);
+          const float2 r1 = rope_rotate(lo[2 * v + 1], hi[2 * v + 1], c[2 * v + 1]);
+          a.w[v] = pack_elems(r0.x, r1.x);
+          b.w[v] = pack_elems(r0.y, r1.y);
+        }
+        elem_t* dst = row0 < r.q_dim
+                          ? r.q_heads + (static_cast<size_t>(row0 / kHd) * T + t) * kHd + i
+                          : r.view.keys + r.view.offset<kPaged>((row0 - r.q_dim) / kHd, position) + i;
+        store16(dst, a);
+        store16(dst + kHalf, b);
       }
-      elem_t* dst = row0 < r.q_dim
-                        ? r.q_heads + (static_cast<size_t>(row0 / kHd) * T + t) * kHd + i
-                        : r.view.keys + r.view.offset<kPaged>((row0 - r.q_dim) / kHd, position) + i;
-      store16(dst, a);
-      store16(dst + kHalf, b);
     }
+  }
+}
+
+// The same for cache rows on 8-byte boundaries only: an item is four pairs of one
+// piece. Kept small (one loop, not unrolled): a second unrolled copy of the
+// above slowed the 192 x 128 tile's aligned calls by 1 %.
+template <bool kPaged, int BW, int BT, int kThreads, class Tile>
+__device__ __forceinline__ void rope_copy_out_narrow(const Tile& tile, const GemmRope& r, int T, int N, int t0,
+                                                     int w0) {
+#pragma unroll 1
+  for (int item = static_cast<int>(threadIdx.x); item < BT * (BW / 64) * 8; item += kThreads) {
+    const int quad = item % 8, row = item / 8 % BT, k = item / (8 * BT);
+    if (t0 + row >= T || w0 + 64 * k >= N) continue;
+    const int byte = (64 * k + 4 * quad) * 2;
+    const uint2 lo_w = *reinterpret_cast<const uint2*>(tile.slot(row, byte));
+    const uint2 hi_w = *reinterpret_cast<const uint2*>(tile.slot(row, byte + 64));
+    const float lo[4] = {elem_lo(lo_w.x), elem_hi(lo_w.x), elem_lo(lo_w.y), elem_hi(lo_w.y)};
+    const float hi[4] = {elem_lo(hi_w.x), elem_hi(hi_w.x), elem_lo(hi_w.y), elem_hi(hi_w.y)};
+    const RopePiece piece = rope_piece(w0 + 64 * k, r.view.head_dim);
+    emit_rope_quad<kPaged>(r, T, t0 + row, piece.row0, piece.i0 + 4 * quad, r.view.head_dim, lo, hi);
   }
 }
 
@@ -529,13 +544,19 @@ __device__ __forceinline__ void store_ring_tile_staged(const mfma_acc4 (&acc)[FW
   if constexpr (!kFp32Out) {
     if (grid.rope.table != nullptr) {
       const GemmRope& r = grid.rope;
-      if (r.view.head_dim == 64) {
+      if (grid.narrow_cache) {
+        if (r.paged) {
+          rope_copy_out_narrow<true, BW, BT, kThreads>(tile, r, T, N, t0, w0);
+        } else {
+          rope_copy_out_narrow<false, BW, BT, kThreads>(tile, r, T, N, t0, w0);
+        }
+      } else if (r.view.head_dim == 64) {
         if (r.paged) {
           rope_copy_out<64, true, BW, BT, kThreads>(tile, r, T, N, t0, w0);
         } else {
           rope_copy_out<64, false, BW, BT, kThreads>(tile, r, T, N, t0, w0);
         }
-      } else if constexpr (BW % 128 == 0) {  // the planner keeps 128-row heads off other tiles
+      } else {
         if (r.paged) {
           rope_copy_out<128, true, BW, BT, kThreads>(tile, r, T, N, t0, w0);
         } else {
@@ -589,7 +610,7 @@ __global__ __launch_bounds__(64 * kWavesW * kWavesT) void gemm_nt_kernel(
   for (int c = 0; c < kPerW; ++c) {
     const int row = w0 + kRowsPerPass * c + trow;
     live |= (row < N ? 1u : 0u) << c;
-    wsrc[c] = W + static_cast<size_t>(weight_row(min(row, N - 1), grid.ffn)) * K + work.k_first;
+    wsrc[c] = W + static_cast<size_t>(weight_row(min(row, N - 1), grid)) * K + work.k_first;
   }
 #pragma unroll
   for (int c = 0; c < kPerT; ++c) {
@@ -664,6 +685,16 @@ __global__ __launch_bounds__(64 * kWavesW * kWavesT) void gemm_nt_kernel(
   }
 
   float* partial = grid.partial != nullptr ? grid.partial + static_cast<size_t>(work.split) * T * N : nullptr;
+  if constexpr (!kFp32Out) {
+    if (grid.rope.table != nullptr && partial == nullptr) {
+      if (grid.rope.paged) {
+        store_rope_tile<FW, FT, true>(acc, grid.rope, T, N, t0 + wt, w0 + ww, col, grp);
+      } else {
+        store_rope_tile<FW, FT, false>(acc, grid.rope, T, N, t0 + wt, w0 + ww, col, grp);
+      }
+      return;
+    }
+  }
   store_gemm_tile<FW, FT, kFp32Out>(acc, Y, partial, T, N, t0 + wt, w0 + ww, col, grp, grid);
 }
 
@@ -697,7 +728,7 @@ constexpr int kRingK = 32;
 //  - 192 x 128, kWaves = 8: wave tiles of 96 x 32 (three 64-row heads per
 //    block tile), so 3072 q/k/v rows and 2048 tokens make exactly 256 tiles;
 //  - 128 x 128, kWaves = 8: wave tiles of 64 x 32, for projections whose
-//    larger tiles would leave compute units idle (two blocks fit a CU);
+//    larger tiles would leave compute units idle;
 //  - 64 x 128, kWaves = 8: wave tiles of 32 x 32, for few tokens, where the
 //    weights' stream and the split partials count more than the matrix rate.
 // kRK: K per ring stage, 32 (64-byte rows) or 64 (128-byte rows: twice the
@@ -750,7 +781,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_ring_kernel(void* __restrict
   for (int i = 0; i < kLoads; ++i) {
     const int row = kLoadRows * (kWaves * i + wave) + lane / kLanesPerRow;
     const int chunk = (lane % kLanesPerRow) ^ row_swizzle(row);
-    src[i] = (row < BW ? W + static_cast<size_t>(weight_row(min(w0 + row, N - 1), grid.ffn)) * K
+    src[i] = (row < BW ? W + static_cast<size_t>(weight_row(min(w0 + row, N - 1), grid)) * K
                            : X + static_cast<size_t>(min(t0 + row - BW, T - 1)) * K) + work.k_first + 8 * chunk;
   }
   const uint32_t ring_base = lds_address_of(ring) + static_cast<uint32_t>(wave * 1024);
@@ -1072,21 +1103,21 @@ struct GemmPlan {
 // fraction of a compute unit's MFMA peak. Splitting K is considered only when
 // the tiles alone leave compute units idle, and costs a reduction: a launch, a
 // part per slice, and the fp32 partials' round trip through memory. The plan
-// depends on the sizes alone, not on the entry, so that every fused entry gives
-// the bits of the plain product.
+// depends on the sizes and the workspace alone, not on the entry, the head size
+// or the destinations' alignment, so that every fused entry sums K in the plain
+// product's slices and gives its bits, and the workspace asked for is the one
+// that any entry's plan uses. (With tiles that the RoPE epilogue of 128-row heads
+// could not take left out of its plan, and the workspace of the plain one, q/k/v
+// of 4096 rows took 44 us at 385 to 512 tokens, 256 x 256 tiles on 32 compute
+// units, where this plan takes 13 to 15.)
 // Fitted to T = 64 .. 1024 over the four projections of a 2048-wide layer,
 // every tile and split forced in turn (o_proj at 256 tokens: 64 x 128 in four
 // slices 13.9 us, 128 x 128 in four 15.2, in eight 18.5; the estimates order
 // them so; before the fill and slice terms eight was chosen). These times
 // are from before the loads were spread over the products, which made every
-// ring tile faster by 2 to 20 %. Each slice
-// keeps at least 256 K and is a whole number of the shape's K stages. With
-// wide_waves, an unsplit plan uses only shapes whose waves own 128 W rows
-// (the RoPE epilogue for 128-row heads). The 192-row tile is for unsplit
-// plans, and without narrow_ok neither it nor the 64-row tile runs unsplit
-// (their RoPE epilogue needs the staged store).
-GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wide_waves = false,
-                   bool narrow_ok = true) {
+// ring tile faster by 2 to 20 %. Each slice keeps at least 256 K and is a whole
+// number of the shape's K stages. The 192-row tile is for unsplit plans.
+GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes) {
   struct Option {
     GemmShape shape;
     int bw, bt, stage_k;
@@ -1123,14 +1154,13 @@ GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes, bool wi
       const int k_chunk = ((K + splits - 1) / splits + o.stage_k - 1) / o.stage_k * o.stage_k;
       if (splits > 1 && k_chunk < 256) break;
       const int used = (K + k_chunk - 1) / k_chunk;
-      if (wide_waves && used == 1 && o.bt != 256) continue;
       // 192-row tiles unsplit only: split four ways for q/k/v at 512 tokens
       // they measured slower than 128 x 128 tiles split in two
-      if (o.bw == 192 && (used > 1 || !narrow_ok)) continue;
+      if (o.bw == 192 && used > 1) continue;
       // 64-row tiles unsplit only once they fill the device: short of that
       // o_proj with its norm at 640 tokens took 20.5 us, against 18.8 with
       // 128 x 128 tiles split in two
-      if (o.bw == 64 && used == 1 && (!narrow_ok || tiles < cus)) continue;
+      if (o.bw == 64 && used == 1 && tiles < cus) continue;
       const size_t bytes = used > 1 ? static_cast<size_t>(used) * T * N * sizeof(float) : 0;
       if (bytes > workspace_bytes) break;
       const long long rounds = (tiles * used + cus - 1) / cus;
@@ -1171,23 +1201,22 @@ void launch_gemm_ring(void* Y, bool fp32_out, const elem_t* X, const elem_t* W, 
   }
 }
 
+// Whether every row of the cache lies on a 16-byte boundary.
+bool aligned_rows(const KvCacheView& v) {
+  return ((reinterpret_cast<uintptr_t>(v.keys) | reinterpret_cast<uintptr_t>(v.values)) & 15u) == 0 &&
+         v.page_stride % 8 == 0 && v.head_stride % 8 == 0;
+}
+
 // Returns whether the residual RMSNorm `norm` was applied (a split plan whose
 // rows the fused reduction covers); otherwise Y holds the projection.
 bool run_gemm(void* Y, bool fp32_out, const elem_t* X, const elem_t* W, int T, int N, int K, void* workspace,
               size_t workspace_bytes, int ffn, hipStream_t s, const GemmRope* rope = nullptr,
               const GemmNorm* norm = nullptr) {
-  const bool wide_waves = rope != nullptr && rope->view.head_dim == 128;
-  // The staged RoPE epilogue's conditions (staged_store_ok), known here.
-  const bool narrow_ok =
-      rope == nullptr ||
-      (rope->view.head_dim == 64 &&
-       ((reinterpret_cast<uintptr_t>(rope->q_heads) | reinterpret_cast<uintptr_t>(rope->view.keys) |
-         reinterpret_cast<uintptr_t>(rope->view.values)) & 15u) == 0 &&
-       rope->view.page_stride % 8 == 0 && rope->view.head_stride % 8 == 0);
-  const GemmPlan plan = plan_gemm(T, N, K, device_compute_units(), workspace != nullptr ? workspace_bytes : 0,
-                                  wide_waves, narrow_ok);
+  const GemmPlan plan = plan_gemm(T, N, K, device_compute_units(), workspace != nullptr ? workspace_bytes : 0);
   GemmGrid grid{(T + plan.bt - 1) / plan.bt, (N + plan.bw - 1) / plan.bw, plan.splits, plan.k_chunk,
                 plan.splits > 1 ? static_cast<float*>(workspace) : nullptr, ffn,
+                rope != nullptr && rope->view.head_dim == 128 && plan.splits == 1 ? 1 : 0,
+                rope != nullptr && !aligned_rows(rope->view) ? 1 : 0,
                 rope != nullptr ? *rope : GemmRope{}};
   switch (plan.shape) {
     case GemmShape::kRing256x256:
