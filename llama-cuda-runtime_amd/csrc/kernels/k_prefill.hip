@@ -1335,7 +1335,7 @@ typedef short lds_v4i16 __attribute__((ext_vector_type(4)));
 template <bool kPaged, int kHeadDim, int kRF, int kKG>
 __global__ __launch_bounds__(256 * kKG, kHeadDim == 64 ? 4 : 2) void flash_prefill_kernel(
     elem_t* __restrict__ out, const elem_t* __restrict__ q_heads, KvCacheView view, int num_heads,
-    int group, int tokens, int start_position, float scale_log2e, bool folded) {
+    int group, int tokens, int start_position, float scale_log2e, int first_round) {
   constexpr int kWaves = 4 * kKG;
   constexpr int kRows = 16 * kRF;                         // query positions per block
   constexpr int kSteps = kHeadDim / 32;                   // MFMA k-steps over head_dim
@@ -1350,25 +1350,29 @@ __global__ __launch_bounds__(256 * kKG, kHeadDim == 64 ? 4 : 2) void flash_prefi
 
   // XCD-aware order: XCD x (block id mod 8) takes the contiguous run of units
   // [x * per, (x + 1) * per) of the kv-head-major order, so one XCD's L2 holds
-  // the keys and values of few kv heads (one, for 8 kv heads). Within a head
-  // the longest rows start first; `folded`, only the longer half does, and the
-  // shorter half follows from the shortest up, so that the two blocks of a
-  // compute unit (dispatched round robin) have the same work in sum.
+  // the keys and values of few kv heads (one, for 8 kv heads), once for every
+  // four query heads of a kv head. Within a head the longest rows come first.
+  // The XCD's compute units take `first_round` blocks in that order; the rest
+  // follow from its other end, so that where all blocks are resident at once, the
+  // second block of a compute unit (dispatched round robin) is the shorter the
+  // longer its first is.
   const int row_blocks = (tokens + kRows - 1) / kRows;
   const int units = row_blocks * view.num_kv_heads;
   const int per_xcd = (units + 7) / 8;
-  const int u = static_cast<int>(blockIdx.x % 8u) * per_xcd + static_cast<int>(blockIdx.x / 8u);
+  const int nth = static_cast<int>(blockIdx.x / 8u);
+  int at = nth < first_round ? nth : static_cast<int>(gridDim.x / 8u) - 1 - (nth - first_round);
+  int quad = 0;
+  for (; at >= per_xcd; at -= per_xcd) ++quad;
+  const int u = static_cast<int>(blockIdx.x % 8u) * per_xcd + at;
   if (u >= units) return;  // the whole block: no barrier has been met
   const int kv = u / row_blocks;
-  const int place = u % row_blocks;
-  const int longer = (row_blocks + 1) / 2;
-  const int r0 = (folded && place >= longer ? place - longer : row_blocks - 1 - place) * kRows;
+  const int r0 = (row_blocks - 1 - u % row_blocks) * kRows;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = lane_id();
   const int col = lane & 15;
   const int grp = lane >> 4;
   const int kg = wave >> 2;  // key group: tiles kg, kg + kKG, ...
-  const int g = blockIdx.z * 4 + (wave & 3);
+  const int g = quad * 4 + (wave & 3);
   const bool active = g < group;
   const int head = kv * group + (active ? g : 0);
 
@@ -1774,28 +1778,41 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_attention_generic_ker
   if (lane + 64 < head_dim) o[lane + 64] = float_to_elem(acc1);
 }
 
+// The two-group blocks of head_dim 64 fit a compute unit twice. When all of them
+// are resident (one to two blocks a unit), the kernel takes the second round in
+// reverse. Against longest first throughout: 39.0 us against 44.5 at T = 2048 (32
+// rows), 88 against 101 at start 2048, 16.0 against 17.3 at T = 1000 (16 rows),
+// with 64 heads on 8 or 16 kv heads 23.4 against 31.8 at T = 1024.
 template <bool kPaged, int kHeadDim, int kRF, int kKG>
 void launch_flash_blocks(elem_t* o, const elem_t* q, const KvCacheView& v, int num_heads, int group,
-                         int tokens, int start_position, float scale_log2e, bool folded, hipStream_t s) {
-  const unsigned zs = static_cast<unsigned>((group + 3) / 4);
+                         int tokens, int start_position, float scale_log2e, hipStream_t s) {
   const int units = (tokens + 16 * kRF - 1) / (16 * kRF) * v.num_kv_heads;
-  const dim3 grid(static_cast<unsigned>((units + 7) / 8 * 8), 1u, zs);
-  flash_prefill_kernel<kPaged, kHeadDim, kRF, kKG><<<grid, 256 * kKG, 0, s>>>(
-      o, q, v, num_heads, group, tokens, start_position, scale_log2e, folded);
+  const int per_xcd = (units + 7) / 8 * ((group + 3) / 4);
+  const int xcd_cus = std::max(1, device_compute_units() / 8);
+  const int first_round = kHeadDim == 64 && kKG == 2 && per_xcd <= 2 * xcd_cus ? xcd_cus : per_xcd;
+  flash_prefill_kernel<kPaged, kHeadDim, kRF, kKG><<<static_cast<unsigned>(per_xcd * 8), 256 * kKG, 0, s>>>(
+      o, q, v, num_heads, group, tokens, start_position, scale_log2e, first_round);
 }
 
 // The block for a chunk (T tokens at a start position, 8 kv heads of 4 query
 // heads, 256 compute units; head_dim 64 unless said; each figure against the
-// other blocks' best):
-//  - 32 rows, two key groups, once that still gives every compute unit two
-//    blocks: a tile's LDS reads serve twice the rows. T = 2048: 44.5 us against
-//    47.2 with 16 rows; at start 2048, 102 against 118. At head_dim 128, where
-//    one block fits a compute unit, 75 against 82.
+// other blocks' best). A tile's LDS reads serve twice the rows in blocks of 32
+// rows, but these are half as many and each twice as long:
+//  - 32 rows, two key groups, where they make nearly two blocks a compute unit,
+//    all resident (7/4 to 2): T = 2048 39.0 us against 42.1 with 16 rows, T = 1792
+//    33.8 against 34.9, equal at T = 1664; and from 7/3 on: T = 2560 57.1 against
+//    60.5. Between, a third round of few blocks costs more: T = 2080 44.8 against
+//    42.9, 31.2 against 26.4 with 16 kv heads of 2 at T = 1040. Behind cached keys
+//    every block is long and the third round fills: from 7/4 on, at start 2048
+//    T = 1792 83 against 100, T = 2240 118 against 136. With one query head a kv
+//    head, two of eight waves work, and a resident round of 32 rows waits on
+//    its longest block: 8 heads, T = 2048, 34.2 against 29.3. At head_dim 128,
+//    where one block fits a compute unit, from two rounds on: 57 against 77.
 //  - 16 rows, four key groups (16 waves), where 16-row blocks leave compute
 //    units with one block or none and the keys are many: T = 500 at 6144,
-//    paged, 75 us against 87; T = 200 at 2000 26 against 30. With few keys the
+//    paged, 65 us against 77; T = 300 at 3000 31 against 37. With few keys the
 //    groups find no tiles (T = 77 at 500: 10.4 against 10.2).
-//  - 16 rows, two key groups otherwise (T = 1024: 17.0 us, 22 with 32 rows).
+//  - 16 rows, two key groups otherwise (T = 1024: 14.9 us, 20.4 with 32 rows).
 template <bool kPaged, int kHeadDim>
 void launch_flash(elem_t* o, const elem_t* q, const KvCacheView& v, int num_heads, int group,
                   int tokens, int start_position, float scale, hipStream_t s) {
@@ -1804,20 +1821,23 @@ void launch_flash(elem_t* o, const elem_t* q, const KvCacheView& v, int num_head
   const long long heads = static_cast<long long>(v.num_kv_heads) * ((group + 3) / 4);
   const long long units32 = (tokens + 31) / 32 * heads;
   const long long units16 = (tokens + 15) / 16 * heads;
-  if (units32 >= 2 * cus) {
-    const bool folded = kHeadDim == 64 && units32 <= 2 * cus;
-    launch_flash_blocks<kPaged, kHeadDim, 2, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e,
-                                                folded, s);
+  bool rows32 = units32 >= 2 * cus;
+  if (kHeadDim == 64) {
+    const bool behind_keys = start_position >= tokens / 2;
+    rows32 = units32 <= 2 * cus ? 4 * units32 >= 7 * cus && (group > 1 || behind_keys)
+                                : 3 * units32 >= 7 * cus || behind_keys;
+  }
+  if (rows32) {
+    launch_flash_blocks<kPaged, kHeadDim, 2, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e, s);
     return;
   }
   if constexpr (kHeadDim == 64) {
     if (units16 <= cus && start_position + tokens >= 1024) {
-      launch_flash_blocks<kPaged, kHeadDim, 1, 4>(o, q, v, num_heads, group, tokens, start_position, scale_log2e,
-                                                  false, s);
+      launch_flash_blocks<kPaged, kHeadDim, 1, 4>(o, q, v, num_heads, group, tokens, start_position, scale_log2e, s);
       return;
     }
   }
-  launch_flash_blocks<kPaged, kHeadDim, 1, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e, false, s);
+  launch_flash_blocks<kPaged, kHeadDim, 1, 2>(o, q, v, num_heads, group, tokens, start_position, scale_log2e, s);
 }
 
 }  // namespace

@@ -17,12 +17,19 @@ pytestmark = pytest.mark.gpu
 
 # (tokens, start, heads, kv heads, head_dim)
 CASES = [
-    (2047, 0, 32, 8, 64), (2049, 0, 32, 8, 64),    # 64 blocks of 32 rows a kv head, and one more
-    (2015, 40, 32, 8, 64), (2016, 0, 16, 8, 128),  # just below: 16 rows
+    (2047, 0, 32, 8, 64), (2049, 0, 32, 8, 64),    # 64 blocks of 32 rows a kv head, and one more (16 rows)
+    (2015, 40, 32, 8, 64), (2016, 0, 16, 8, 128),  # just below: 16 rows at head_dim 128
     (2048, 0, 16, 8, 128),
     (511, 513, 32, 8, 64), (512, 512, 32, 8, 64), (513, 512, 32, 8, 64),  # four groups up to one block a unit
     (500, 523, 32, 8, 64), (500, 524, 32, 8, 64),  # and from 1024 keys on
     (1, 1023, 32, 8, 64), (17, 2000, 16, 2, 64), (65, 0, 8, 8, 64), (33, 1500, 16, 8, 128),
+    # the second resident round in reverse: one to two blocks a unit, runs of several and of less than one kv head,
+    # two blocks of four heads a kv head (one of them half empty), empty places at the end of the last XCD
+    (1009, 0, 64, 8, 64), (1000, 0, 32, 16, 64), (1024, 0, 16, 16, 64), (700, 0, 32, 4, 64), (530, 9, 48, 8, 64),
+    (600, 0, 10, 10, 64),
+    # 32 rows from 7/4 blocks a unit on, with one head a kv head only behind cached keys, and again from 7/3 on
+    (1761, 0, 32, 8, 64), (1760, 0, 32, 8, 64), (1024, 512, 16, 16, 64), (1024, 511, 16, 16, 64), (1185, 0, 32, 16, 64),
+    (1217, 0, 32, 16, 64),
 ]
 
 
