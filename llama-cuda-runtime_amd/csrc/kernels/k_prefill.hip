@@ -142,7 +142,7 @@ struct GemmGrid {
   int k_chunk;
   float* partial;  // nullptr: no split, write Y
   int ffn;         // > 0: gated (Y is act[T][ffn], N == 2 * ffn)
-  int half_heads;  // rows in the pieces of 128-row heads (unsplit RoPE launches)
+  int half_heads;  // 1: rows in the pieces of 128-row heads (unsplit RoPE launches)
   // RoPE: the cache's rows lie on 8-byte boundaries only. Here and not behind
   // `rope`, whose arguments arrive later: read there by the epilogue, 2048 tokens
   // of 3072 rows took 0.4 us longer.
@@ -152,8 +152,8 @@ struct GemmGrid {
 
 __device__ __forceinline__ int weight_row(int p, const GemmGrid& g) {
   if (g.ffn > 0) return (((p >> 5) << 4) | (p & 15)) + ((p & 16) ? g.ffn : 0);
-  if (g.half_heads) return (p & ~127) + ((p & 64) >> 1) + (p & 31) + ((p & 32) << 1);
-  return p;
+  // half_heads: bits 5 and 6 change places
+  return p ^ (96 * (((p >> 5) ^ (p >> 6)) & g.half_heads));
 }
 
 __device__ __forceinline__ float swiglu_rounded(float gate, float up) {
@@ -652,6 +652,9 @@ __global__ __launch_bounds__(64 * kWavesW * kWavesT) void gemm_nt_kernel(
   fetch(0);
   deposit(0);
   __syncthreads();
+  // The loop starts on a 64-byte line: off it, T = 2048, N = 2048, K = 2080 takes
+  // 39.5 us instead of 38.3.
+  asm volatile(".p2align 6");
   for (int s = 0; s < stages; ++s) {
     const int buf = s & 1;
     if (s + 1 < stages) fetch((s + 1) * kStageK);
