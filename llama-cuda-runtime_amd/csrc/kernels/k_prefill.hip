@@ -950,7 +950,7 @@ constexpr int kRing128x128Stages = 4;
 // a CU). With 77 tokens, cold weights, against the 128 x 128 tile's best split:
 // down 15.4 us (18.2), q/k/v 11.5 (14.0), o_proj 10.6 (12.2), each with its
 // reduction; four or six stages, or 128 K a stage, measured no faster.
-constexpr double kRing64x128Efficiency = 0.20;
+constexpr double kRing64x128Efficiency = 0.22;
 constexpr int kRing64x128K = 64;
 constexpr int kRing64x128Stages = 3;
 // Waves per ring block. Eight (two per SIMD) measured faster than four with
@@ -1113,13 +1113,14 @@ struct GemmPlan {
 // could not take left out of its plan, and the workspace of the plain one, q/k/v
 // of 4096 rows took 44 us at 385 to 512 tokens, 256 x 256 tiles on 32 compute
 // units, where this plan takes 13 to 15.)
-// Fitted to T = 64 .. 1024 over the four projections of a 2048-wide layer,
-// every tile and split forced in turn (o_proj at 256 tokens: 64 x 128 in four
-// slices 13.9 us, 128 x 128 in four 15.2, in eight 18.5; the estimates order
-// them so; before the fill and slice terms eight was chosen). These times
-// are from before the loads were spread over the products, which made every
-// ring tile faster by 2 to 20 %. Each slice keeps at least 256 K and is a whole
-// number of the shape's K stages. The 192-row tile is for unsplit plans.
+// Fitted to T = 64 .. 2048 over the four projections of a 2048-wide layer and
+// those of 3072- and 4096-wide ones, every tile and split forced in turn, with
+// weights from HBM. The 64-row tile's efficiency and the cost of a slice decide
+// where few tokens change from the 128-row tile in many slices to the 64-row
+// tile in half as many: down at 160 tokens takes 22.8 us with 128 x 128 in eight,
+// 21.3 with 64 x 128 in four (weights cached 22.2 and 17.9); q/k/v at 192 15.2
+// in four, 14.0 in two. Each slice keeps at least 256 K and is a whole number
+// of the shape's K stages. The 192-row tile is for unsplit plans.
 GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes) {
   struct Option {
     GemmShape shape;
@@ -1146,7 +1147,7 @@ GemmPlan plan_gemm(int T, int N, int K, int cus, size_t workspace_bytes) {
   constexpr double kCuPeak = 9.8e12;     // bf16 dense flop/s per compute unit
   constexpr double kBandwidth = 5.0e12;  // sustained bytes/s for the partials' round trip
   constexpr double kReduce = 3e-6;
-  constexpr double kSlice = 0.5e-6;
+  constexpr double kSlice = 0.7e-6;
   GemmPlan best{GemmShape::k128x128, 128, 128, 1, K, 0};
   double best_time = -1.0;
   for (const Option& o : options) {
