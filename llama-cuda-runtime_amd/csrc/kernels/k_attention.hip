@@ -158,20 +158,27 @@ int launch_waves(int group, const DecodeArgs& a) {
   return launch_blocks<kPaged, kHeadDim, kHeads, kAttnWaves, false>(group, a);
 }
 
-// From this many splits on, one block serves up to four query heads of a kv
-// head, reading each key and value once for them. Below, per-head blocks fill
-// the device better: 11 splits (3000 positions) take 11.0 us per head against
-// 12.2 shared at head_dim 64, 11.8 against 12.3 at 128; 16 splits (4096) 11.5
-// against 10.6 and 13.2 against 11.3; 64 splits (32768, paged) 52.5 against
-// 26.6 and 51.1 against 38.2.
-constexpr int kSharedHeadsMinSplits = 16;
+// One block serves up to four query heads of a kv head, reading each key and
+// value once for them, where per-head blocks would read 40 MB or more (their
+// reads of one kv head come from L2, at about 5 TB/s in all) and the shared
+// blocks still give every second compute unit one. Per head against shared, 32
+// query heads on 8, head_dim 64 unless said: 16 splits of 4096 positions (34 MB)
+// 7.9 us against 10.2, 19 of 5000 (41 MB) 13.1 against 12.3, 32 of 8192 (67 MB)
+// 17.1 against 11.7; head_dim 128, 16 of 3000 (49 MB) 18.4 against 14.0; 16 query
+// heads, 32 of 8192 (34 MB) 9.4 against 10.0, 32 of 16384 16.0 against 11.4. Of
+// too few blocks: 8 query heads on 2, 16 of 32768 (67 MB, 32 shared blocks) 16.7
+// against 23.8, 64 splits (128) 16.3 against 13.8.
+constexpr long long kSharedHeadsElements = 10 * 1000 * 1000;  // of keys, four bytes each with their values
+constexpr int kSharedBlocksMin = 128;
 
 template <bool kPaged, int kHeadDim, int kGroup>
 int launch_decode(const DecodeArgs& a) {
   constexpr int kShared = kGroup < 4 ? kGroup : 4;
-  const int status = kShared > 1 && a.splits >= kSharedHeadsMinSplits
-                         ? launch_waves<kPaged, kHeadDim, kShared>(kGroup, a)
-                         : launch_waves<kPaged, kHeadDim, 1>(kGroup, a);
+  const bool shared = kShared > 1 &&
+                      static_cast<long long>(a.num_heads) * kHeadDim * a.seq_len >= kSharedHeadsElements &&
+                      a.num_heads / kShared * a.splits >= kSharedBlocksMin;
+  const int status = shared ? launch_waves<kPaged, kHeadDim, kShared>(kGroup, a)
+                            : launch_waves<kPaged, kHeadDim, 1>(kGroup, a);
   if (status != LCR_OK) return status;
   if (a.splits > 1) {
     merge_splits_kernel<<<a.num_heads, kMergeThreads, 0, a.stream>>>(a.out, a.partials, a.splits, kHeadDim);
